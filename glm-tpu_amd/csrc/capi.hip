@@ -103,20 +103,35 @@ bool uses_decode_path(int64_t routes, int64_t hidden, int64_t intermediate) {
   return routes <= kMaxDecodeRoutes && decode_path_fits(hidden, intermediate);
 }
 
-// Whether the bf16 down projection keeps tall stripes (512 weight rows a work
-// item) for about `listings` route tiles: unless its work items would leave
-// most CUs of the last round idle where 256-row stripes (twice the items)
-// fill the rounds -- an expert-parallel share's few experts (32 tiles x 12
-// tall stripes = 384 items on 256 CUs: 1.5 rounds).
-bool down_tall_fills(int64_t listings, int64_t hidden) {
+// Whether a bf16 prefill layer runs on tall stripes (512 weight rows a work
+// item, every wide tile listed twice) rather than 256-row ones.  Tall stripes
+// read each activation fragment for twice the MFMAs, but halve the number of
+// work items.  They run where
+//   * both projections can take them: 256-row stripes skip a wide tile's second
+//     listing, and a skipped workgroup still takes its turn in the round-robin
+//     over the shader engines, so that every other engine idles (64 experts, H
+//     2560, I 640, T=2000: 392 -> 324 us without; H 1536, I 1152, T=4000: 641
+//     -> 537);
+//   * experts see 16 routes on average: below that the items are weight
+//     streams of one column group, and fewer, longer ones are slower (GLM-5
+//     shape, T=9 / 64 / 256: +7 / +3.5 / +1 %; from 16 to 48 routes an expert
+//     the two are within 2 %, evenly popular experts slightly for 256-row
+//     stripes, skewed ones for tall; T=2048: tall 2266, 256-row 2291 us);
+//   * the gate/up items fill 2.5 rounds of the CUs, so that the last round
+//     costs little (32 of 256 experts, one or two rounds: T=2048 / 4000 tall
+//     361 / 528 us, 256-row 314 / 500; 64 of 256, two to three rounds: 583 /
+//     833, 543 / 864).  An expert has at least one listing, a skewed routing
+//     about 1.5 listings per 128 routes.
+bool bf16_tall_stripes(int64_t routes, int64_t global_experts, int64_t experts, int64_t hidden,
+                       int64_t intermediate) {
+  if (routes < 16 * global_experts || intermediate % prefill_tall_bn(2) != 0 || hidden % prefill_tall_bn(1) != 0)
+    return false;
   int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-                                               hipSuccess || cus <= 0)
-    return true;
-  auto fill = [&](int64_t items) { return (double)items / (double)(((items + cus - 1) / cus) * cus); };
-  const int64_t tall_items = listings * (hidden / prefill_tall_bn(1));
-  const int64_t short_items = listings * (hidden / prefill_bn(1));
-  return !(fill(tall_items) < 0.85 && fill(short_items) > fill(tall_items) + 0.1);
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  const int64_t listings = std::max(experts, routes * experts / global_experts * 3 / 256);
+  return 2 * listings * (intermediate / prefill_tall_bn(2)) >= 5 * (int64_t)cus;
 }
 
 // Byte layout of the glm_moe_routed_experts workspace.
@@ -370,16 +385,15 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
                           prefill_fits(hidden_size, intermediate, 1) && prefill_rows_fit(tokens, hidden_size) &&
                           prefill_rows_fit(n, intermediate);
   const int tile_rows = wide_tiles ? prefill_wide_tile_rows() : gemm_shape_rows(shape);
-  // Tall stripes (512 weight rows a work item) pay where experts see enough
-  // routes to fill a few column groups: GLM-5 shape, T=1024 / 2048 layer
-  // -3 / -5 %, T=512 even, but T=9 / 16 / 64 / 256 +7 / +7 / +3.5 / +1 %, so
-  // they run from 16 routes per expert on average.  Where a projection runs
-  // on them, its wide tiles run as two work items per stripe, one per 256-row
-  // half: the plan lists each tile of more than half the tile rows twice.  At
-  // most ceil(c / 128) listings per expert of c routes: within L.max_tiles.
-  const bool tall = n >= 16 * (int64_t)global_experts;  // routes per expert of the whole layer
-  const bool wide_twice = tall && wide_tiles &&
-                          (intermediate % prefill_tall_bn(2) == 0 || hidden_size % prefill_tall_bn(1) == 0);
+  // Tall stripes: bf16_tall_stripes(); in the FP8 mode from 16 routes per
+  // expert on average (32 .. 256 experts, T=256 .. 2048: -2 .. -18 % against
+  // 256-row stripes), on each projection that N allows.  On bf16 tall stripes
+  // a wide tile runs as two work items per stripe, one per 256-row half: the
+  // plan lists each tile of more than half the tile rows twice.  At most
+  // ceil(c / 128) listings per expert of c routes: within L.max_tiles.
+  const bool tall = fp8 ? n >= 16 * (int64_t)global_experts  // routes per expert of the whole layer
+                        : wide_tiles && bf16_tall_stripes(n, global_experts, num_experts, hidden_size, intermediate);
+  const bool wide_twice = tall && wide_tiles;
   const int32_t max_tiles =
       (int32_t)max_tiles_for(n, num_experts, wide_twice ? tile_rows / 2 : tile_rows);  // <= L.max_tiles
   p.tile_rows = tile_rows;
@@ -493,12 +507,7 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
   d.stripe_run = prefill_stripe_run(1);
   d.tile_rows = tile_rows;
   d.wide_twice = p.wide_twice;
-  // about one tile per expert of the call, or its share of the routes in whole tiles
-  // (wide tiles counted as their two listings)
-  const int64_t listing_rows = p.wide_twice ? tile_rows / 2 : tile_rows;
-  const int64_t listings_est =
-      std::max<int64_t>(num_experts, (n * num_experts / global_experts + listing_rows - 1) / listing_rows);
-  d.tall = tall && (fp8 || down_tall_fills(listings_est, hidden_size)) ? 1 : 0;
+  d.tall = g.tall;
   timer.arm(kStageDown);
   GLM_HIP(launch_grouped_gemm(d, shape, 1, kEpiStoreBf16, stream), "down launch");
   timer.done(kStageDown);

@@ -428,9 +428,8 @@ __global__ __launch_bounds__(64 * WAVES, 1) void prefill_gemm_kernel(const Group
   }
   tile += t0;
   if (stripe < 0 || stripe >= stripes || tile >= a.max_tiles) return;
-  // A wide tile listed twice: on tall stripes each listing takes one 256-row
-  // half of the stripe, as predicted above; 256-row stripes take the whole
-  // stripe on the first listing and skip the second.
+  // A wide tile listed twice (tall stripes only): each listing takes one
+  // 256-row half of the stripe, as predicted above.
   const bool listing_ok = BLOCK == kStripeBlockBytes
                               ? it.half == 0
                               : (wide_half < 0 ? it.live <= kBM && it.half == 0
@@ -1490,6 +1489,8 @@ hipError_t launch_grouped_gemm_prefill(const GroupedGemmArgs& a, int tables, int
   // the FP8 kernel's tiles: at most 128 routes, each listed once
   if (a.xq != nullptr && (a.tile_rows > kBM || a.wide_twice != 0)) return hipErrorInvalidValue;
   if (!prefill_fits(a.n, a.k, tables) || !prefill_rows_fit(a.x_rows, a.k)) return hipErrorInvalidValue;
+  // a list that names wide tiles twice is for tall stripes
+  if (a.wide_twice != 0 && (a.tall == 0 || a.n % prefill_tall_bn(tables) != 0)) return hipErrorInvalidValue;
   if ((a.outq != nullptr) != (a.outq_scale != nullptr)) return hipErrorInvalidValue;
   if (a.outq != nullptr && !prefill_quantizes_output(a, tables, epilogue)) return hipErrorInvalidValue;
   if (a.xq != nullptr) {

@@ -612,13 +612,10 @@ def _routes_with_counts(counts, tokens, top_k, seed):
 # FP8 mode plans the same routes in tiles of 128.
 # I = 256 gives the down projection K = 2 blocks (the weight ring's first
 # blocks are the whole K loop), I = 1024 eight.
-# Stripes: a projection whose N is a multiple of 512 (down: H) or 256 (gate/up:
-# I) runs tall stripes (512 weight rows a work item), where a wide tile is
-# listed twice and each listing takes half the stripe; otherwise 256-row
-# stripes, which skip the second listing.  H = 1536 / I = 256, 1024: both
-# projections tall; H = 768 / I = 384: neither; H = 1536 / I = 384: gate/up on
-# 256-row stripes beside a tall down projection (the list holds second
-# listings that the gate/up kernel skips).
+# Stripes: the bf16 layers here are too small for tall stripes
+# (test_bf16_tall_stripes_match_oracle runs those); the FP8 projections whose N
+# is a multiple of 512 (down: H) or 256 (gate/up: I) run tall ones: H = 1536 /
+# I = 256, 1024 both, H = 768 / I = 384 neither, H = 1536 / I = 384 down alone.
 WIDE_COUNTS = [129, 150, 170, 190, 200, 220, 230, 256, 300, 513, 600, 700, 1, 40, 128, 17]
 
 
@@ -649,6 +646,33 @@ def test_prefill_wide_tiles_match_oracle(device, activations, hidden, inter, see
     assert bool(ok) and ref_ok
     close = assert_moe_close if activations == "bfloat16" else assert_fp8_close
     print(cfg, activations, close(host_f32(out), ref))
+
+
+# Tall stripes of the bf16 kernel: from 16 routes per expert and 2.5 rounds of
+# gate/up items on 256 CUs, listings (1.5 per 128 routes, at least one per
+# expert) x I / 256.  32 experts with WIDE_COUNTS, I = 2304: 75 x 9 = 675 items,
+# wide tiles of every column-group count as two listings (gate/up K = 4 blocks,
+# down K = 18).  64 experts of ~125 routes, I = 1792: 93 x 7 = 651, tiles of 5 ..
+# 8 column groups and wide ones.  128 experts of 16, I = 1280: 128 x 5 = 640,
+# tiles of one or two groups; one token fewer runs 256-row stripes.
+@pytest.mark.parametrize("tokens,experts,hidden,inter,counts", [
+    (800, 32, 512, 2304, True), (1000, 64, 512, 1792, False), (256, 128, 512, 1280, False),
+    (255, 128, 512, 1280, False),
+])
+def test_bf16_tall_stripes_match_oracle(device, tokens, experts, hidden, inter, counts):
+    from glm_moe.layers.moe.routed_experts import routed_experts
+
+    cfg, x, ids, w, tables = _small_case(tokens, experts, hidden, inter, 8, 0.0, seed=tokens + 3)
+    if counts:
+        rest = tokens * 8 - sum(WIDE_COUNTS)
+        more = experts - len(WIDE_COUNTS)
+        ids, w = _routes_with_counts(WIDE_COUNTS + [rest // more + (i < rest % more) for i in range(more)], tokens, 8,
+                                     seed=5)
+    t = _device_tables(tables, device)
+    out, ok = routed_experts(bf16_dev(x, device), dev(ids, device), dev(w, device), *(t[k] for k in TABLE_KEYS))
+    ref, ref_ok = O.routed_experts(x, ids, w, **tables)
+    assert bool(ok) and ref_ok
+    print(cfg, assert_moe_close(host_f32(out), ref))
 
 
 def test_routed_experts_invalid_routes_follow_reference(device):
