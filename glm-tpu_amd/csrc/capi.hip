@@ -103,6 +103,15 @@ bool uses_decode_path(int64_t routes, int64_t hidden, int64_t intermediate) {
   return routes <= kMaxDecodeRoutes && decode_path_fits(hidden, intermediate);
 }
 
+// Compute units of the current device.
+int compute_units() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    return 256;
+  return cus;
+}
+
 // Whether a bf16 prefill layer runs on tall stripes (512 weight rows a work
 // item, every wide tile listed twice) rather than 256-row ones.  Tall stripes
 // read each activation fragment for twice the MFMAs, but halve the number of
@@ -126,12 +135,38 @@ bool bf16_tall_stripes(int64_t routes, int64_t global_experts, int64_t experts, 
                        int64_t intermediate) {
   if (routes < 16 * global_experts || intermediate % prefill_tall_bn(2) != 0 || hidden % prefill_tall_bn(1) != 0)
     return false;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
   const int64_t listings = std::max(experts, routes * experts / global_experts * 3 / 256);
-  return 2 * listings * (intermediate / prefill_tall_bn(2)) >= 5 * (int64_t)cus;
+  return 2 * listings * (intermediate / prefill_tall_bn(2)) >= 5 * (int64_t)compute_units();
+}
+
+// Panels of the reference's kernel: 32 rows.
+constexpr int kPanelRows = 32;
+// Whether a panel matmul runs on the prefill kernel: its geometry fits, and
+// there is enough work that the time goes there and not into the call (m n k
+// of 2^29: 72 rows over 60 of 256 experts, N 6144, K 2048, 1.6 times faster;
+// 480 rows of N 1024, K 256 take the few us of a launch either way, and the
+// call without a workspace is the shorter one).
+bool panel_matmul_on_tiles(int64_t m, int64_t k, int32_t groups, int64_t n) {
+  return m > 0 && k > 0 && groups > 0 && n > 0 && prefill_fits(n, k, 1) && prefill_rows_fit(m, k) &&
+         m * k >= ((int64_t)1 << 29) / n;
+}
+// Its stripes, by bf16_tall_stripes' rule for one table.
+bool panel_tall_stripes(int64_t rows, int64_t groups, int64_t n) {
+  return rows >= 16 * groups && n % prefill_tall_bn(1) == 0 &&
+         2 * std::max(groups, rows * 3 / 256) * (n / prefill_tall_bn(1)) >= 5 * (int64_t)compute_units();
+}
+// Its workspace: runs of panels, tile descriptors, tile count.
+struct PanelLayout {
+  size_t run_ends, tile_desc, tile_count, total;
+};
+PanelLayout panel_layout(int64_t capacity) {
+  PanelLayout L{};
+  size_t off = 0;
+  L.run_ends = off;   off = align_up(off + sizeof(int32_t) * 2 * (size_t)capacity);
+  L.tile_desc = off;  off = align_up(off + sizeof(int32_t) * 4 * (size_t)capacity);
+  L.tile_count = off; off = align_up(off + sizeof(int32_t));
+  L.total = off;
+  return L;
 }
 
 // Byte layout of the glm_moe_routed_experts workspace.
@@ -721,6 +756,23 @@ int glm_moe_panel_fp8_matmul(const uint16_t* lhs, int64_t m, int64_t k, const ui
                              const int32_t* panel_live_counts, const int32_t* active_panels,
                              int32_t capacity, const uint8_t* owned_rows, const uint8_t* valid,
                              int32_t result_dtype, void* out, void* stream) {
+  return glm_moe_panel_fp8_matmul_ws(lhs, m, k, weight_bits, scale, groups, n, panel_expert_ids, panel_row_starts,
+                                     panel_live_counts, active_panels, capacity, owned_rows, valid, result_dtype, out,
+                                     nullptr, 0, stream);
+}
+
+size_t glm_moe_panel_fp8_matmul_workspace_bytes(int64_t m, int64_t k, int32_t groups, int64_t n) {
+  if (!panel_matmul_on_tiles(m, k, groups, n)) return 0;
+  return panel_layout((m + kPanelRows - 1) / kPanelRows + groups - 1).total;
+}
+
+int glm_moe_panel_fp8_matmul_ws(const uint16_t* lhs, int64_t m, int64_t k, const uint8_t* weight_bits,
+                                const float* scale, int32_t groups, int64_t n,
+                                const int32_t* panel_expert_ids, const int32_t* panel_row_starts,
+                                const int32_t* panel_live_counts, const int32_t* active_panels,
+                                int32_t capacity, const uint8_t* owned_rows, const uint8_t* valid,
+                                int32_t result_dtype, void* out, void* workspace, size_t workspace_bytes,
+                                void* stream) {
   GLM_REQUIRE(m > 0 && k > 0 && groups > 0 && n > 0, "panel FP8 geometry/dtypes disagree with M32/N256/K128");
   GLM_REQUIRE(k % 128 == 0 && n % 256 == 0 && n / 128 <= 128, "panel FP8 geometry/dtypes disagree with M32/N256/K128");
   GLM_REQUIRE(capacity == (m + 31) / 32 + groups - 1, "panel FP8 geometry/dtypes disagree with M32/N256/K128");
@@ -731,7 +783,7 @@ int glm_moe_panel_fp8_matmul(const uint16_t* lhs, int64_t m, int64_t k, const ui
               "null tensor pointer");
   hipStream_t s = as_stream(stream);
   const int64_t elem = result_dtype == GLM_MOE_F32 ? 4 : 2;
-  GLM_HIP(launch_zero_rows(out, m, n * elem, owned_rows, valid, s), "zero launch");
+  const int epilogue = result_dtype == GLM_MOE_F32 ? kEpiStoreF32 : kEpiStoreBf16;
   GroupedGemmArgs g{};
   g.experts = groups;
   g.rows = (int32_t)m;
@@ -743,17 +795,56 @@ int glm_moe_panel_fp8_matmul(const uint16_t* lhs, int64_t m, int64_t k, const ui
   g.s0 = scale;
   g.n = (int32_t)n;
   g.k = (int32_t)k;
+  g.max_tiles = capacity;
+  g.out = out;
+  g.ldo = n;
+  g.table_stride = 0;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(lhs) | reinterpret_cast<uintptr_t>(weight_bits) |
+                         reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(workspace)) & 15) == 0;
+  if (workspace != nullptr && aligned && panel_matmul_on_tiles(m, k, groups, n)) {
+    // the panels as tiles of up to 256 rows on the pipelined prefill kernel:
+    // an expert's weights are streamed once per 256 rows instead of once per
+    // panel (a layer body of three such calls, 256 experts, H 6144, I 2048: 500
+    // tokens 2974 -> 1655 us, 2000 tokens 6923 -> 2579 us, FP32 down rows)
+    const PanelLayout L = panel_layout(capacity);
+    if (workspace_bytes < L.total)
+      return fail(GLM_MOE_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", L.total, workspace_bytes);
+    char* ws = static_cast<char*>(workspace);
+    PanelTilesArgs t{};
+    t.expert_ids = panel_expert_ids;
+    t.row_starts = panel_row_starts;
+    t.live_counts = panel_live_counts;
+    t.active = active_panels;
+    t.valid = valid;
+    t.owned = owned_rows;
+    t.capacity = capacity;
+    t.panel_rows = kPanelRows;
+    t.experts = groups;
+    t.rows = (int32_t)m;
+    t.tile_rows = prefill_wide_tile_rows();
+    const bool tall = panel_tall_stripes(m, groups, n);
+    t.wide_twice = tall ? 1 : 0;
+    t.run_ends = reinterpret_cast<int32_t*>(ws + L.run_ends);
+    t.tile_desc = reinterpret_cast<int32_t*>(ws + L.tile_desc);
+    t.tile_count = reinterpret_cast<int32_t*>(ws + L.tile_count);
+    t.out = out;
+    t.row_bytes = n * elem;
+    GLM_HIP(launch_panel_tiles(t, s), "panel tiles launch");
+    g.tile_desc = t.tile_desc;
+    g.tile_count = t.tile_count;
+    g.tile_rows = t.tile_rows;
+    g.wide_twice = t.wide_twice;
+    g.tall = tall ? 1 : 0;
+    GLM_HIP(launch_grouped_gemm_prefill(g, 1, epilogue, s), "panel matmul launch");
+    return GLM_MOE_OK;
+  }
+  GLM_HIP(launch_zero_rows(out, m, n * elem, owned_rows, valid, s), "zero launch");
   g.tile_expert = panel_expert_ids;
   g.tile_row = panel_row_starts;
   g.tile_live = panel_live_counts;
   g.tile_count = active_panels;
-  g.max_tiles = capacity;
   g.valid = valid;
-  g.out = out;
-  g.ldo = n;
-  g.table_stride = 0;
-  GLM_HIP(launch_grouped_gemm(g, kShapePanel32, 1, result_dtype == GLM_MOE_F32 ? kEpiStoreF32 : kEpiStoreBf16, s),
-          "panel matmul launch");
+  GLM_HIP(launch_grouped_gemm(g, kShapePanel32, 1, epilogue, s), "panel matmul launch");
   return GLM_MOE_OK;
 }
 

@@ -265,16 +265,49 @@ template <int NCG, int RGS, int TABLES, int EPI, int WAVES>
 __device__ __forceinline__ void store_tile_lines(const GroupedGemmArgs& a, uint8_t* lds,
                                                  const f32x4 (&acc)[TABLES][RGS][NCG], const int (&orow)[NCG],
                                                  int live, int wave, int lane, int64_t n_item) {
-  static_assert(EPI == kEpiSwiglu || EPI == kEpiStoreBf16, "the prefill epilogues store bf16");
+  static_assert(EPI == kEpiSwiglu || EPI == kEpiStoreBf16 || (EPI == kEpiStoreF32 && TABLES == 1),
+                "the prefill epilogues store bf16, or the FP32 sums of one table");
+  constexpr int EL = EPI == kEpiStoreF32 ? 4 : 2;  // bytes of an output
   constexpr int OUT = WAVES * RGS * 16;  // outputs of one route row in this work item
   constexpr int ROWS = NCG * 16;
-  constexpr int PITCH = OUT * 2 + 16;    // staged row bytes: +16 puts a fragment's 16 rows in distinct banks
-  constexpr int LPR = OUT * 2 / 16;      // 16-byte pieces of a route row
-  static_assert(ROWS * PITCH + ROWS * 4 <= kPrefillLds, "the staged tile fits the LDS");
+  constexpr int PITCH = OUT * EL + 16;   // staged row bytes: +16 puts a fragment's 16 rows in distinct banks
+  constexpr int LPR = OUT * EL / 16;     // 16-byte pieces of a route row
+  // column groups staged at a time: all of them, or (FP32 outputs of large
+  // tiles) as many as the LDS holds
+  constexpr int FIT = (kPrefillLds - ROWS * 4) / (16 * PITCH);
+  constexpr int CH = NCG < FIT ? NCG : FIT;
+  static_assert(CH >= 1 && (EL == 4 || CH == NCG), "the staged tile fits the LDS");
   static_assert((LPR & (LPR - 1)) == 0, "pieces per row: a power of two");
   const int lrow = lane & 15, lgrp = lane >> 4;
-  int* const srow = reinterpret_cast<int*>(lds + ROWS * PITCH);
+  int* const srow = reinterpret_cast<int*>(lds + CH * 16 * PITCH);
   __syncthreads();  // every wave is done with the rings
+  if (wave == 0 && lgrp == 0) {
+#pragma unroll
+    for (int cg = 0; cg < NCG; ++cg) srow[cg * 16 + lrow] = (int)out_row(a, cg * 16 + lrow, live, orow[cg]);
+  }
+  if constexpr (EPI == kEpiStoreF32) {
+    float* const out = static_cast<float*>(a.out) + n_item;
+#pragma unroll
+    for (int c0 = 0; c0 < NCG; c0 += CH) {
+      if (c0 > 0) __syncthreads();  // the pass before is stored
+#pragma unroll
+      for (int cg = c0; cg < (c0 + CH < NCG ? c0 + CH : NCG); ++cg)
+#pragma unroll
+        for (int rg = 0; rg < RGS; ++rg)
+          *reinterpret_cast<f32x4*>(lds + ((cg - c0) * 16 + lrow) * PITCH +
+                                    (wave * RGS * 16 + rg * 16 + lgrp * 4) * 4) = acc[0][rg][cg];
+      __syncthreads();
+      const int rows = (c0 + CH < NCG ? CH : NCG - c0) * 16;
+      for (int i = wave * 64 + lane; i < rows * LPR; i += WAVES * 64) {
+        const int r = i / LPR, part = i % LPR;
+        const int o = srow[c0 * 16 + r];
+        if (o >= 0)
+          __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(lds + r * PITCH + part * 16),
+                                      reinterpret_cast<u32x4*>(out + (int64_t)o * a.ldo + part * 4));
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int cg = 0; cg < NCG; ++cg)
 #pragma unroll
@@ -288,10 +321,6 @@ __device__ __forceinline__ void store_tile_lines(const GroupedGemmArgs& a, uint8
       *reinterpret_cast<u32x2*>(lds + (cg * 16 + lrow) * PITCH + (wave * RGS * 16 + rg * 16 + lgrp * 4) * 2) =
           u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
     }
-  if (wave == 0 && lgrp == 0) {
-#pragma unroll
-    for (int cg = 0; cg < NCG; ++cg) srow[cg * 16 + lrow] = (int)out_row(a, cg * 16 + lrow, live, orow[cg]);
-  }
   __syncthreads();
   if constexpr (EPI == kEpiSwiglu && OUT % kScaleBlock == 0) {
     if (a.outq != nullptr) {
@@ -1513,6 +1542,9 @@ hipError_t launch_grouped_gemm_prefill(const GroupedGemmArgs& a, int tables, int
   if (tables == 1 && epilogue == kEpiStoreBf16)
     return tall_list && a.n % prefill_tall_bn(1) == 0 ? launch_prefill<1, 4, 8, kEpiStoreBf16>(a, stream)
                                                       : launch_prefill<1, 2, 8, kEpiStoreBf16>(a, stream);
+  if (tables == 1 && epilogue == kEpiStoreF32)
+    return tall_list && a.n % prefill_tall_bn(1) == 0 ? launch_prefill<1, 4, 8, kEpiStoreF32>(a, stream)
+                                                      : launch_prefill<1, 2, 8, kEpiStoreF32>(a, stream);
   return hipErrorInvalidValue;
 }
 

@@ -188,6 +188,31 @@ struct PanelPlanArgs {
 };
 hipError_t launch_panel_plan(const PanelPlanArgs& a, hipStream_t stream);
 
+// The prefill kernels' work list of a panel plan, and the plan's zero rows:
+// runs of consecutive panels of one expert over consecutive rows become tiles
+// of up to tile_rows rows (whatever the panels name, each valid panel's rows
+// are in exactly one tile of its expert), heaviest run first.
+struct PanelTilesArgs {
+  const int32_t* expert_ids;   // [capacity] the panels
+  const int32_t* row_starts;
+  const int32_t* live_counts;
+  const int32_t* active;       // [1]
+  const uint8_t* valid;        // [1]: 0: no tiles, every row zero
+  const uint8_t* owned;        // [rows]: 0: a row to zero
+  int32_t capacity;
+  int32_t panel_rows;
+  int32_t experts;
+  int32_t rows;
+  int32_t tile_rows;
+  int32_t wide_twice;
+  int32_t* run_ends;           // workspace [2][capacity]: a run's first and last panel
+  int32_t* tile_desc;          // [capacity][4], 16-byte aligned
+  int32_t* tile_count;         // [1]
+  void* out;                   // [rows] rows of row_bytes (a multiple of 16)
+  int64_t row_bytes;
+};
+hipError_t launch_panel_tiles(const PanelTilesArgs& a, hipStream_t stream);
+
 // Owned decode slots as one-row tiles (kernel.py:185-191 slot compaction).
 hipError_t launch_slot_tiles(const int32_t* local_ids, const uint8_t* owned, int32_t slots,
                              int32_t experts, int32_t* tile_expert, int32_t* tile_row,

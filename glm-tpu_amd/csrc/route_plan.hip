@@ -513,6 +513,78 @@ __global__ __launch_bounds__(kPlanThreads) void panel_plan_kernel(const PanelPla
   }
 }
 
+// A panel whose rows the projection computes (any other computes nothing).
+__device__ __forceinline__ bool panel_ok(const PanelTilesArgs& a, int p) {
+  const int e = a.expert_ids[p], r = a.row_starts[p], live = a.live_counts[p];
+  return e >= 0 && e < a.experts && r >= 0 && live > 0 && live <= a.panel_rows && r <= a.rows - live;
+}
+// Whether panel p > 0 goes on where panel p - 1 ends: same expert, next rows.
+__device__ __forceinline__ bool panel_follows(const PanelTilesArgs& a, int p) {
+  return panel_ok(a, p - 1) && a.live_counts[p - 1] == a.panel_rows && a.expert_ids[p] == a.expert_ids[p - 1] &&
+         a.row_starts[p] == a.row_starts[p - 1] + a.panel_rows;
+}
+
+// Workgroup 0 lists the tiles; the others zero the rows no panel owns, four
+// rows a wave (a row's flag is read before any of its bytes is written, so a
+// plan that owns every row costs its flags).  Latency-bound, one launch where
+// the zeroing alone was one: 11 us a call at 4000 rows of 4-12 KB when every
+// thread looked up the flag of its own dword.
+__global__ __launch_bounds__(kPlanThreads) void panel_tiles_kernel(const PanelTilesArgs a) {
+  __shared__ int s_scan[kPlanWaves + 1];
+  __shared__ int s_free[3 * kPlanThreads];
+  const int tid = threadIdx.x;
+  const bool valid = a.valid[0] != 0;
+  if (blockIdx.x > 0) {
+    const int lane = tid & 63;
+    const int64_t words = a.row_bytes / 16;
+    for (int j = 0; j < 4; ++j) {
+      const int64_t r = ((int64_t)(blockIdx.x - 1) * kPlanWaves + (tid >> 6)) * 4 + j;
+      if (r >= a.rows || (valid && a.owned[r] != 0)) continue;
+      u32x4* const row = reinterpret_cast<u32x4*>(static_cast<uint8_t*>(a.out) + r * a.row_bytes);
+      for (int64_t i = lane; i < words; i += 64) row[i] = u32x4{0u, 0u, 0u, 0u};
+    }
+    return;
+  }
+  const int active = valid ? min(max(a.active[0], 0), a.capacity) : 0;
+  int* const first = a.run_ends;
+  int* const last = a.run_ends + a.capacity;
+  int runs = 0;
+  for (int base = 0; base < active; base += kPlanThreads) {
+    const int p = base + tid;
+    const bool ok = p < active && panel_ok(a, p);
+    const bool head = ok && !(p > 0 && panel_follows(a, p));
+    int total = 0;
+    const int before = block_exclusive_scan(head ? 1 : 0, s_scan, &total);
+    if (head) first[runs + before] = p;
+    if (ok && !(p + 1 < active && panel_ok(a, p + 1) && panel_follows(a, p + 1)))
+      last[runs + before + (head ? 1 : 0) - 1] = p;
+    runs += total;
+  }
+  __syncthreads();  // first and last are this workgroup's own writes
+  if (runs > kPlanThreads) {
+    // a plan of very many runs (no build_expert_panels plan: those have one
+    // run an expert): a tile per panel
+    for (int p = tid; p < active; p += kPlanThreads)
+      *reinterpret_cast<int4*>(a.tile_desc + 4 * (int64_t)p) =
+          panel_ok(a, p) ? make_int4(a.expert_ids[p], p, a.row_starts[p], a.live_counts[p]) : make_int4(-1, 0, 0, 0);
+    if (tid == 0) a.tile_count[0] = active;
+    return;
+  }
+  int e = 0, start = 0, count = 0;
+  if (tid < runs) {
+    const int f = first[tid], l = last[tid];
+    e = a.expert_ids[f];
+    start = a.row_starts[f];
+    count = (l - f) * a.panel_rows + a.live_counts[l];
+  }
+  const int nt = tid < runs ? tiles_of_count(count, a.tile_rows, a.wide_twice) : 0;
+  int total = 0;
+  const int t0 = heavy_first_tile(count, nt, runs, s_free, s_scan, &total);
+  for (int i = 0; i < nt; ++i)
+    *reinterpret_cast<int4*>(a.tile_desc + 4 * (int64_t)(t0 + i)) = make_int4(e, t0, start, count);
+  if (tid == 0) a.tile_count[0] = total;
+}
+
 // Owned slots first, in slot order, as one-row tiles; ids clipped to [0, E).
 __global__ void slot_tiles_kernel(const int32_t* ids, const uint8_t* owned, int slots, int experts,
                                   int32_t* tile_expert, int32_t* tile_row, int32_t* tile_live,
@@ -617,6 +689,14 @@ hipError_t launch_route_plan_from_logits(const RoutePlanArgs& a, const RouterPas
 hipError_t launch_panel_plan(const PanelPlanArgs& a, hipStream_t stream) {
   label_next_launch("build_expert_panels_r%d_g%d_p%d", a.rows, a.groups, a.panel_rows);
   return launch_kernel(panel_plan_kernel, dim3(1), dim3(kPlanThreads), 0, stream, a);
+}
+
+hipError_t launch_panel_tiles(const PanelTilesArgs& a, hipStream_t stream) {
+  // a listing covers at least one panel (a tile listed twice more than four):
+  // never more than capacity of them
+  if (a.panel_rows <= 0 || a.tile_rows < 8 * a.panel_rows || a.row_bytes % 16 != 0) return hipErrorInvalidValue;
+  const int64_t zero_blocks = ((int64_t)a.rows + 4 * kPlanWaves - 1) / (4 * kPlanWaves);
+  return launch_kernel(panel_tiles_kernel, dim3((unsigned)(1 + zero_blocks)), dim3(kPlanThreads), 0, stream, a);
 }
 
 hipError_t launch_slot_tiles(const int32_t* local_ids, const uint8_t* owned, int32_t slots,

@@ -54,6 +54,11 @@ SIGNATURES: dict[str, tuple] = {
         ctypes.c_int,
         [_vp, _i64, _i64, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _vp, _vp],
     ),
+    "glm_moe_panel_fp8_matmul_workspace_bytes": (_sz, [_i64, _i64, _i32, _i64]),
+    "glm_moe_panel_fp8_matmul_ws": (
+        ctypes.c_int,
+        [_vp, _i64, _i64, _vp, _vp, _i32, _i64, _vp, _vp, _vp, _vp, _i32, _vp, _vp, _i32, _vp, _vp, _sz, _vp],
+    ),
     "glm_moe_routed_projection_workspace_bytes": (_sz, [_i32]),
     "glm_moe_routed_projection": (
         ctypes.c_int,

@@ -3,9 +3,10 @@
 Mirrors ``prefill_panel_fp8_matmul`` of
 ``glm_tpu/kernels/fp8_grouped_matmul/panel_kernel.py:31-153``: sorted bf16
 rows against their panel's local expert, weights decoded per 128x128 block to
-bf16, FP32 accumulation in ascending K blocks.  On the GPU the panels are the
-work list of the grouped gfx950 kernel: the kernel reads the sorted rows in
-place (no packed copy), and unowned rows / invalid plans produce zeros.
+bf16, FP32 accumulation in ascending K blocks.  On the GPU runs of an expert's
+panels become the tiles of the pipelined gfx950 prefill kernel (geometries that
+it does not take run panel by panel): the rows are read in place (no packed
+copy), and unowned rows / invalid plans produce zeros.
 """
 
 from __future__ import annotations
@@ -55,12 +56,14 @@ def prefill_panel_fp8_matmul(
         raise ValueError("panel FP8 geometry/dtypes disagree with M32/N256/K128")
     _lib.require_device(lhs, weight_bits, scale, panels.expert_ids, panels.row_starts, panels.live_counts)
     out = torch.empty((m, n), dtype=dtype, device=lhs.device)
+    nbytes = _lib.lib().glm_moe_panel_fp8_matmul_workspace_bytes(m, k, groups, n)
+    workspace = torch.empty(nbytes, dtype=torch.uint8, device=lhs.device) if nbytes else None
     _lib.call(
-        "glm_moe_panel_fp8_matmul",
+        "glm_moe_panel_fp8_matmul_ws",
         _lib.ptr(lhs), m, k, _lib.ptr(weight_bits), _lib.ptr(scale), groups, n,
         _lib.ptr(panels.expert_ids), _lib.ptr(panels.row_starts), _lib.ptr(panels.live_counts),
         _lib.ptr(panels.active_panels), panels.expert_ids.numel(), _lib.ptr(panels.owned_rows),
         _lib.ptr(panels.valid), _lib.F32 if dtype == torch.float32 else _lib.BF16, _lib.ptr(out),
-        _lib.stream_of(lhs),
+        _lib.ptr(workspace), nbytes, _lib.stream_of(lhs),
     )
     return out, panels.valid

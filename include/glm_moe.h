@@ -137,6 +137,21 @@ int glm_moe_panel_fp8_matmul(const uint16_t* lhs, int64_t m, int64_t k, const ui
                              int32_t capacity, const uint8_t* owned_rows, const uint8_t* valid,
                              int32_t result_dtype, void* out, void* stream);
 
+/* The same with a workspace of glm_moe_panel_fp8_matmul_workspace_bytes bytes,
+ * where the call lists runs of an expert's panels as tiles of up to 256 rows,
+ * so that its weights are read once per tile instead of once per panel.  The
+ * size is 0 (and a workspace is not looked at) for calls that run panel by panel:
+ * k above 8192, m x k bf16 of 2 GiB and more, m n k below 2^29; so do pointers
+ * not 16-byte aligned and a NULL workspace, as in glm_moe_panel_fp8_matmul. */
+size_t glm_moe_panel_fp8_matmul_workspace_bytes(int64_t m, int64_t k, int32_t groups, int64_t n);
+int glm_moe_panel_fp8_matmul_ws(const uint16_t* lhs, int64_t m, int64_t k, const uint8_t* weight_bits,
+                                const float* scale, int32_t groups, int64_t n,
+                                const int32_t* panel_expert_ids, const int32_t* panel_row_starts,
+                                const int32_t* panel_live_counts, const int32_t* active_panels,
+                                int32_t capacity, const uint8_t* owned_rows, const uint8_t* valid,
+                                int32_t result_dtype, void* out, void* workspace, size_t workspace_bytes,
+                                void* stream);
+
 /* Replaces glm_tpu/kernels/fp8_grouped_matmul/kernel.py:125-299 fp8_routed_projection:
  * one bf16 row per route slot lhs [slots, k] against the slot's expert
  * (ids clipped to [0, experts)) in 1 or 2 tables; out [slots, tables, n] f32 or bf16;

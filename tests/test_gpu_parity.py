@@ -271,6 +271,68 @@ def test_panel_matmul_closed_form_and_invalid_plan(device):
         assert bool(ok) == (offset == 2)
 
 
+# Panels as tiles of up to 256 rows: an expert's run of panels ends in every
+# way (one row, one panel, a tile and a row, exact tiles), with unowned experts
+# before and after; 20 experts x 16384 outputs fill 2.5 rounds of 512-row
+# stripes (wide tiles listed twice, FP32 tiles staged in passes); K = 8320 is
+# past the prefill kernel (panel by panel).
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("counts,offset,local,n,k", [
+    ([5, 300, 33, 1, 513, 64, 31, 0, 256, 40], 1, 8, 768, 640),
+    ([600, 130, 256, 1, 17, 90] + [40] * 14, 0, 20, 16384, 128),
+    ([7, 70, 300], 0, 3, 256, 8320),
+])
+def test_panel_matmul_tiles_match_oracle(device, dtype, counts, offset, local, n, k):
+    from glm_moe.kernels.fp8_grouped_matmul.panel_kernel import prefill_panel_fp8_matmul
+    from glm_moe.kernels.fp8_grouped_matmul.panels import build_expert_panels
+
+    rng = np.random.default_rng(n + k)
+    m = sum(counts)
+    x = O.bf16_round(rng.normal(0, 0.2, (m, k)).astype(np.float32))
+    bits = torch.from_numpy(rng.normal(0, 0.15, (local, n, k)).astype(np.float32)).to(
+        torch.float8_e4m3fn).view(torch.uint8).numpy()
+    scales = rng.uniform(0.1, 2.0, (local, n // 128, k // 128)).astype(np.float32)
+    c = np.array(counts, np.int32)
+    plan = build_expert_panels(dev(c, device), torch.tensor(offset, dtype=torch.int32, device=device), rows=m,
+                               local_groups=local)
+    got, ok = prefill_panel_fp8_matmul(bf16_dev(x, device), dev(bits, device), dev(scales, device), plan,
+                                       result_dtype=dtype)
+    ref, _ = O.panel_fp8_matmul(x, bits, scales, O.build_expert_panels(c, offset, rows=m, local_groups=local),
+                                result_dtype="float32")
+    assert bool(ok)
+    # FP32 sums of K products in another order: each within K eps of the sum of
+    # their magnitudes, far inside it in practice (eps sqrt(K) of the row's scale)
+    atol = 8 * 2**-24 * np.sqrt(k) * np.abs(ref).max()
+    got = host_f32(got)
+    np.testing.assert_allclose(got, ref, rtol=1e-5 if dtype == torch.float32 else 2**-8, atol=atol)
+    rows = np.arange(m)
+    owned = (rows >= c[:offset].sum()) & (rows < c[:offset + local].sum())
+    np.testing.assert_array_equal(got[~owned], 0)
+
+
+@pytest.mark.parametrize("panels", [20, 1100])  # broken runs: listed by run; more runs than one pass lists: by panel
+def test_panel_matmul_takes_panels_in_any_order(device, panels):
+    from glm_moe.kernels.fp8_grouped_matmul.panel_kernel import prefill_panel_fp8_matmul
+    from glm_moe.kernels.fp8_grouped_matmul.panels import build_expert_panels
+
+    g = torch.Generator(device=device).manual_seed(panels)
+    m, n, k = 32 * panels, 256, 4096
+    x = torch.randn((m, k), generator=g, device=device).to(torch.bfloat16)
+    w = torch.randint(0, 120, (2, n, k), generator=g, device=device, dtype=torch.int32).to(torch.uint8)
+    s = torch.rand((2, n // 128, k // 128), generator=g, device=device)
+    plan = build_expert_panels(torch.tensor([m - 96, 96], dtype=torch.int32, device=device),
+                               torch.tensor(0, dtype=torch.int32, device=device), rows=m, local_groups=2)
+    ref, _ = prefill_panel_fp8_matmul(x, w, s, plan)
+    live = int(plan.active_panels)
+    back = {f: torch.cat([getattr(plan, f)[:live].flip(0), getattr(plan, f)[live:]]).contiguous()
+            for f in ("expert_ids", "row_starts", "live_counts")}
+    got, ok = prefill_panel_fp8_matmul(x, w, s, plan._replace(**back))
+    assert bool(ok) and torch.equal(got, ref)
+    bad = plan._replace(expert_ids=torch.where(plan.row_starts == 32, 9, plan.expert_ids).to(torch.int32))
+    got, _ = prefill_panel_fp8_matmul(x, w, s, bad)  # a panel of no expert computes nothing, the others theirs
+    assert torch.equal(got[:32], ref[:32]) and torch.equal(got[64:], ref[64:])
+
+
 # ----------------------------------------------------------------------------- routed projection
 @pytest.mark.parametrize("tables", [1, 2])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
