@@ -241,6 +241,28 @@ __global__ __launch_bounds__(256) void route_noaux_tc_kernel(const float* logits
   }
 }
 
+// Per-row serving health of a layer routed from logits (router.py:161-166 and
+// the caller's router_valid & grouped_valid, decoder_layer.py:146): the row's
+// logits, the bias and the row's route weights are finite and the layer is
+// healthy.  One wave per row, one launch: as isfinite / all / and tensor
+// operations the same took 16 launches of ~5 us each.
+__global__ __launch_bounds__(256) void route_row_health_kernel(const float* logits, int64_t tokens, int32_t experts,
+                                                               const float* bias, const float* weights,
+                                                               int32_t top_k, const uint8_t* layer_valid,
+                                                               uint8_t* row_valid) {
+  const int lane = threadIdx.x & 63;
+  const int64_t t = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+  if (t >= tokens) return;
+  bool ok = layer_valid[0] != 0;
+  for (int e = lane; e < experts; e += 64) {
+    ok &= isfinite(logits[t * experts + e]);
+    if (bias != nullptr) ok &= isfinite(bias[e]);
+  }
+  if (lane < top_k) ok &= isfinite(weights[t * top_k + lane]);
+  const bool all = __ballot(!ok) == 0;
+  if (lane == 0) row_valid[t] = all ? 1 : 0;
+}
+
 // Wave-wide maximum (every lane active), wave-uniform: the 16-lane row maxima
 // by DPP moves (row16_max_f32), then the four of them through v_readlane -- no
 // LDS round trip.
@@ -527,6 +549,16 @@ hipError_t launch_route_noaux_tc(const float* logits, int64_t tokens, int32_t ex
                          experts, bias, top_k, ids, weights);
   return launch_kernel(route_noaux_tc_kernel<kMaxExperts / 64>, dim3((unsigned)blocks), dim3(256), 0, stream,
                        logits, tokens, experts, bias, top_k, ids, weights);
+}
+
+hipError_t launch_route_row_health(const float* logits, int64_t tokens, int32_t experts, const float* bias,
+                                   const float* weights, int32_t top_k, const uint8_t* layer_valid,
+                                   uint8_t* row_valid, hipStream_t stream) {
+  if (tokens <= 0) return hipSuccess;
+  if (experts <= 0 || top_k <= 0 || top_k > kWave) return hipErrorInvalidValue;
+  label_next_launch("route_row_health_t%lld_e%d", (long long)tokens, experts);
+  return launch_kernel(route_row_health_kernel, dim3((unsigned)((tokens + 3) / 4)), dim3(256), 0, stream, logits,
+                       tokens, experts, bias, weights, top_k, layer_valid, row_valid);
 }
 
 hipError_t launch_quantize_rows_fp8(const uint16_t* x, int64_t rows, int64_t k, uint8_t* q, float* scales,

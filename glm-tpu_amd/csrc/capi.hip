@@ -642,6 +642,20 @@ int glm_moe_route_noaux_tc(const float* router_logits, int64_t tokens, int32_t n
   return GLM_MOE_OK;
 }
 
+int glm_moe_route_row_health(const float* router_logits, int64_t tokens, int32_t num_experts,
+                             const float* correction_bias, const float* route_weights, int32_t top_k,
+                             const uint8_t* layer_valid, uint8_t* row_valid, void* stream) {
+  GLM_REQUIRE(tokens >= 0, "router_logits must have shape [tokens, experts]");
+  GLM_REQUIRE(num_experts > 0 && top_k > 0 && top_k <= num_experts && top_k <= kWave,
+              "top_k must be in [1, min(num_experts, %d)]", kWave);
+  if (tokens == 0) return GLM_MOE_OK;
+  GLM_REQUIRE(router_logits && route_weights && layer_valid && row_valid, "null tensor pointer");
+  GLM_HIP(launch_route_row_health(router_logits, tokens, num_experts, correction_bias, route_weights, top_k,
+                                  layer_valid, row_valid, as_stream(stream)),
+          "row health launch");
+  return GLM_MOE_OK;
+}
+
 int glm_moe_count_nonfinite_fp8(const uint8_t* bits, int64_t n, uint64_t* count, void* stream) {
   GLM_REQUIRE(n >= 0, "byte count must be >= 0");
   if (n == 0) return GLM_MOE_OK;

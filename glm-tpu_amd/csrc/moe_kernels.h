@@ -408,6 +408,11 @@ hipError_t launch_count_nonfinite_fp8(const uint8_t* bits, int64_t n, unsigned l
                                       hipStream_t stream);
 hipError_t launch_route_noaux_tc(const float* logits, int64_t tokens, int32_t experts, const float* bias,
                                  int32_t top_k, int32_t* ids, float* weights, hipStream_t stream);
+// row_valid[t] = *layer_valid and every logit of row t, bias (nullable) and
+// route weight of row t is finite (top_k <= 64).
+hipError_t launch_route_row_health(const float* logits, int64_t tokens, int32_t experts, const float* bias,
+                                   const float* weights, int32_t top_k, const uint8_t* layer_valid,
+                                   uint8_t* row_valid, hipStream_t stream);
 // Per (row, 128-wide block): scale = amax / 448 (1 for an all-zero block),
 // q = e4m3fn(clamp(x / scale, +-448)) rounded to nearest even.  The scales go
 // to scales[kb * n_pos + pos] for each pos = positions[row * per_row + j]

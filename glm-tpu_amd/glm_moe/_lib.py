@@ -41,6 +41,7 @@ SIGNATURES: dict[str, tuple] = {
     "glm_moe_decode_fp8_table": (ctypes.c_int, [_vp, _vp, _i64, _i64, _i32, _i32, _vp, _vp]),
     "glm_moe_swiglu_bf16": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp]),
     "glm_moe_route_noaux_tc": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i32, _vp, _vp, _vp]),
+    "glm_moe_route_row_health": (ctypes.c_int, [_vp, _i64, _i32, _vp, _vp, _i32, _vp, _vp, _vp]),
     "glm_moe_count_nonfinite_fp8": (ctypes.c_int, [_vp, _i64, _vp, _vp]),
     "glm_moe_group_routes": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "glm_moe_group_routes_workspace_bytes": (_sz, [_i64, _i32, _i32]),

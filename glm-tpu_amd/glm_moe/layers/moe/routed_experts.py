@@ -568,19 +568,21 @@ def _shared_expert(hidden: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, d
 
 def _check_layer_shapes(hidden_local, route_indices, route_weights, gate_bits, up_bits, down_bits,
                         contract: GlmMoeNumericalContract, *, rows_exact: int | None) -> None:
+    """The layer bodies' geometry (routes None: the body routes the rows itself)."""
     if hidden_local.ndim != 2 or hidden_local.shape[0] <= 0 or hidden_local.dtype != torch.bfloat16:
         raise ValueError("MoE requires BF16 live rows")
     if rows_exact is not None and hidden_local.shape[0] != rows_exact:
         raise ValueError("grouped MoE input must contain one live row")
     if hidden_local.shape[1] != contract.hidden_size:
         raise ValueError("MoE hidden size differs from contract")
-    expected = (hidden_local.shape[0], contract.top_k)
-    if tuple(route_indices.shape) != expected or tuple(route_weights.shape) != expected:
-        raise ValueError("routing geometry differs from contract")
-    if route_indices.dtype != torch.int32:
-        raise ValueError("routes must be int32")
-    if route_weights.dtype != torch.float32:
-        raise ValueError("route weights must be FP32")
+    if route_indices is not None:
+        expected = (hidden_local.shape[0], contract.top_k)
+        if tuple(route_indices.shape) != expected or tuple(route_weights.shape) != expected:
+            raise ValueError("routing geometry differs from contract")
+        if route_indices.dtype != torch.int32:
+            raise ValueError("routes must be int32")
+        if route_weights.dtype != torch.float32:
+            raise ValueError("route weights must be FP32")
     gate_shape = (contract.local_experts, contract.intermediate_size, contract.hidden_size)
     if tuple(gate_bits.shape) != gate_shape or tuple(up_bits.shape) != gate_shape:
         raise ValueError("expert gate/up geometry differs from contract")
@@ -694,9 +696,9 @@ def prefill_moe_from_router_logits(
     The reference's prefill MLP from the logits on (``decoder_layer.py:123-146``):
     the noaux_tc selection of ``prefill_router`` (``router.py:146``, i.e.
     ``route_glm_noaux_tc_logits``) feeding ``prefill_moe_from_routes``, in one
-    library call (``glm_moe_moe_layer_from_router_logits``; one row: the decode
-    kernels with the resident shared expert, routing inside the gate/up
-    kernel).  ``valid`` is per row, as the
+    library call (``glm_moe_moe_layer_from_router_logits``; up to 8 rows on the
+    decode kernels with the resident shared expert, one row routed inside the
+    gate/up kernel).  ``valid`` is per row, as the
     reference's ``router_valid & grouped_valid``: the layer's health and, per
     row, finite logits, bias and route weights (``router.py:161-166``; the
     hidden rows' own finiteness check belongs to the router's matmul, before
@@ -710,8 +712,7 @@ def prefill_moe_from_router_logits(
         raise ValueError(f"router_logits must have shape {(hidden_local.shape[0], contract.num_experts)}")
     top_k = contract.top_k
     inter, h = contract.intermediate_size, contract.hidden_size
-    ids_probe = torch.zeros((hidden_local.shape[0], top_k), dtype=torch.int32, device=hidden_local.device)
-    _check_layer_shapes(hidden_local, ids_probe, ids_probe.float(), expert_gate_bits_local, expert_up_bits_local,
+    _check_layer_shapes(hidden_local, None, None, expert_gate_bits_local, expert_up_bits_local,
                         expert_down_bits_local, contract, rows_exact=None)
     if contract.fp8_block_shape != (128, 128):
         raise ValueError("expert panels require checkpoint scale blocks128x128")
@@ -719,14 +720,14 @@ def prefill_moe_from_router_logits(
     if (tuple(tables[0].shape) != (inter, h) or tuple(tables[1].shape) != (inter, h)
             or tuple(tables[2].shape) != (h, inter)):
         raise ValueError("prefill shared expert geometry differs from contract")
-    bias = (torch.zeros(contract.num_experts, dtype=torch.float32, device=hidden_local.device)
-            if correction_bias is None else correction_bias)
-    if hidden_local.shape[0] == 1 and contract.num_experts <= 256 and uses_decode_kernels(1, top_k, h, inter):
+    rows = hidden_local.shape[0]
+    logits = router_logits.float().contiguous()
+    bias = None if correction_bias is None else correction_bias.float().contiguous()
+    decode = rows <= RESIDENT_ROWS_MAX and uses_decode_kernels(rows, top_k, h, inter)
+    if decode and rows == 1 and contract.num_experts <= 256:
         # one row: the resident shared expert inside the two decode kernels, which also route
         experts = contract.num_experts
         resident = tuple(t.contiguous() for t in tables)
-        logits = router_logits.float().contiguous()
-        bias = bias.float().contiguous()
         _lib.require_device(hidden_local, logits, bias, expert_gate_bits_local, expert_gate_scale_local,
                             expert_up_bits_local, expert_up_scale_local, expert_down_bits_local,
                             expert_down_scale_local, *resident)
@@ -743,15 +744,33 @@ def prefill_moe_from_router_logits(
             *(_lib.ptr(t) for t in resident), inter, float(contract.routed_scaling_factor), _lib.ptr(ids),
             _lib.ptr(weights), _lib.ptr(out), _lib.ptr(layer_valid), _lib.ptr(ws), ws.numel(),
             _lib.stream_of(hidden_local))
+    elif decode and rows > 1 and correction_bias is not None and tuple(correction_bias.shape) == (
+            contract.num_experts,):
+        # a few rows: the router kernel, then the decode kernels with the resident
+        # shared expert (its weights streamed once per group of up to 4 rows)
+        from glm_moe.layers.moe.router import route_glm_noaux_tc_logits
+
+        ids, weights = route_glm_noaux_tc_logits(logits, bias, top_k=top_k)
+        out, layer_valid = routed_experts(
+            hidden_local, ids, weights, expert_gate_bits_local, expert_gate_scale_local, expert_up_bits_local,
+            expert_up_scale_local, expert_down_bits_local, expert_down_scale_local, route_sum="float32",
+            check_weights=True, routed_scale=contract.routed_scaling_factor,
+            shared_tables=tuple(t.contiguous() for t in tables))
     else:
         out, layer_valid, ids, weights = routed_experts_from_router_logits(
-            hidden_local, router_logits, bias, expert_gate_bits_local, expert_gate_scale_local,
+            hidden_local, logits, bias, expert_gate_bits_local, expert_gate_scale_local,
             expert_up_bits_local, expert_up_scale_local, expert_down_bits_local, expert_down_scale_local,
             top_k=top_k, route_sum="float32", check_weights=True, shared=_shared_expert(hidden_local, *tables),
             routed_scale=contract.routed_scaling_factor)
-    row_valid = (torch.isfinite(router_logits).all(dim=1) & torch.isfinite(bias).all()
-                 & torch.isfinite(weights).all(dim=1))
-    return out, ids, weights, row_valid & layer_valid
+    if (torch.float64 in (router_logits.dtype, None if bias is None else correction_bias.dtype)
+            or (bias is not None and bias.numel() != contract.num_experts)):
+        # a finite FP64 logit may be infinite in FP32
+        row_valid = torch.isfinite(router_logits).all(dim=1) & torch.isfinite(weights).all(dim=1) & layer_valid
+        return out, ids, weights, row_valid if bias is None else row_valid & torch.isfinite(correction_bias).all()
+    row_valid = torch.empty(rows, dtype=torch.bool, device=hidden_local.device)
+    _lib.call("glm_moe_route_row_health", _lib.ptr(logits), rows, contract.num_experts, _lib.ptr(bias),
+              _lib.ptr(weights), top_k, _lib.ptr(layer_valid), _lib.ptr(row_valid), _lib.stream_of(hidden_local))
+    return out, ids, weights, row_valid
 
 
 def moe_grouped_routes(

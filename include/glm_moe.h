@@ -89,6 +89,15 @@ int glm_moe_route_noaux_tc(const float* router_logits, int64_t tokens, int32_t n
                            const float* correction_bias, int32_t top_k, int32_t* route_indices,
                            float* route_weights, void* stream);
 
+/* Per-row health of a layer routed from logits, the reference's router_valid &
+ * grouped_valid (glm_tpu/layers/moe/router.py:161-166,
+ * glm_tpu/models/glm_moe_dsa/decoder_layer.py:146): row_valid[t] = *layer_valid
+ * and the row's logits, the bias (nullable) and the row's route weights
+ * [tokens, top_k] are finite.  top_k <= min(64, experts). */
+int glm_moe_route_row_health(const float* router_logits, int64_t tokens, int32_t num_experts,
+                             const float* correction_bias, const float* route_weights, int32_t top_k,
+                             const uint8_t* layer_valid, uint8_t* row_valid, void* stream);
+
 /* Replaces glm_tpu/layers/moe/routed_experts.py:139-164 group_prefill_routes:
  * sorted_flat_ids = argsort(flat ids, stable), inverse_permutation, group_sizes
  * = bincount (invalid ids count as expert 0), *valid = all ids in [0, E) and no

@@ -1489,6 +1489,53 @@ def test_prefill_moe_from_router_logits_composes_router_and_layer(device):
             assert ok.all() == bool(ref_ok)
 
 
+@pytest.mark.parametrize("tokens,dtype,biased", [(2, torch.float32, True), (8, torch.float32, False),
+                                                 (5, torch.float64, True), (9, torch.bfloat16, True),
+                                                 (70, torch.float32, False)])
+def test_prefill_moe_from_router_logits_row_health(device, tokens, dtype, biased):
+    """Few rows equal router + layer bit for bit, and a row's health is the
+    layer's and its own logits', weights' and the bias's finiteness, for every
+    logit type (a finite FP64 logit stays finite)."""
+    from glm_moe import synthetic as S
+    from glm_moe.contracts import single_gpu_contract
+    from glm_moe.layers.moe.routed_experts import prefill_moe_from_router_logits, prefill_moe_from_routes
+    from glm_moe.layers.moe.router import route_glm_noaux_tc_logits
+
+    experts, h, inter = 70, 512, 256
+    cfg = S.MoeConfig("row-health", tokens, experts, h, inter, 6)
+    x = bf16_dev(S.hidden_states(cfg, 9), device)
+    dt = _device_tables(S.host_expert_tables(cfg, 9), device)
+    tabs = [dt[k] for k in TABLE_KEYS]
+    shared = tuple(bf16_dev((np.random.default_rng(3).standard_normal(s) * 0.05).astype(np.float32), device)
+                   for s in ((inter, h), (inter, h), (h, inter)))
+    contract = single_gpu_contract(hidden_size=h, intermediate_size=inter, num_experts=experts, top_k=6)
+    logits = torch.from_numpy(S.router_logits(cfg, 9)).to(device=device, dtype=dtype)
+    bias = (torch.randn(experts, generator=torch.Generator().manual_seed(1)) * 0.1).to(device) if biased else None
+    zero = torch.zeros(experts, device=device)
+
+    def both(logits, bias):
+        out, ids, w, ok = prefill_moe_from_router_logits(x, logits, bias, *tabs, *shared, contract=contract)
+        ref_ids, ref_w = route_glm_noaux_tc_logits(logits, zero if bias is None else bias, top_k=6)
+        ref, layer_ok = prefill_moe_from_routes(x, ref_ids, ref_w, *tabs, *shared, contract=contract)
+        assert torch.equal(ids, ref_ids) and torch.equal(w.isnan(), ref_w.isnan())
+        want = logits.isfinite().all(1) & ref_w.isfinite().all(1) & layer_ok
+        want = want if bias is None else want & bias.isfinite().all()
+        assert ok.dtype == torch.bool and torch.equal(ok, want)
+        return out, ref, ok
+
+    if dtype == torch.float64:
+        logits[0, 4] = 1e300
+    out, ref, ok = both(logits, bias)
+    assert torch.equal(out, ref) and bool(ok.all())
+    bad = logits.clone()
+    bad[tokens - 1, experts - 1] = -float("inf")  # a finite sigmoid: the other rows stay healthy
+    assert both(bad, bias)[2].tolist() == [True] * (tokens - 1) + [False]
+    if biased:
+        over = bias.clone()
+        over[experts - 1] = float("inf")
+        assert not bool(both(logits, over)[2].any())
+
+
 # ----------------------------------------------------------------------------- few-row shared expert
 @pytest.mark.parametrize("tokens,hidden,inter", [(1, 512, 256), (2, 768, 384), (4, 6144, 2048), (8, 1024, 512)])
 def test_shared_expert_rows_matches_oracle(device, tokens, hidden, inter):
