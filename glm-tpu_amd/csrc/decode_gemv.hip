@@ -257,11 +257,15 @@ __device__ __forceinline__ void gemv_fma(const GemvStream<TABLES, NR>& g, const 
   }
 }
 
-// Straight-line stream of exactly NSTEPS steps, DEPTH in flight: with no loop
+// Straight-line stream of exactly NSTEPS steps, DEPTH in flight (gemv_run: every
+// count from 2 to 8 that the registers allow; one step, K of at most 1024, stays
+// with the loop: its instance made the two-table kernels spill): with no loop
 // back-edge the compiler counts outstanding loads exactly and waits only for
 // the step it is about to multiply.  Order of issue: activation staging
 // loads, the first DEPTH weight steps, then the staging stores (which wait
-// for the activations only).
+// for the activations only).  Against the loop below, layers of 128 experts:
+// H 5120, I 1536 (5 and 6 steps a wave) T=4 148 -> 126 us; H 3072, I 1280 (3
+// and 5) T=6 152 -> 111; H 7168, I 1792 (7) T=1 88.6 -> 69.8.
 template <int NSTEPS, int DEPTH, bool DMA, int TABLES, int NR, int QN>
 __device__ __forceinline__ void gemv_run_fixed(const GemvStream<TABLES, NR>& g, int lane,
                                                float (&acc)[TABLES][QN][NR]) {
@@ -342,8 +346,11 @@ __device__ __forceinline__ void gemv_run(const GemvStream<TABLES, NR>& g, int la
   if (!half) {
     switch (n) {
       case 2: gemv_run_fixed<2, DEPTH, DMA>(g, lane, acc); return;
+      case 3: gemv_run_fixed<3, DEPTH, DMA>(g, lane, acc); return;
       case 4: gemv_run_fixed<4, DEPTH, DMA>(g, lane, acc); return;
+      case 5: gemv_run_fixed<5, DEPTH, DMA>(g, lane, acc); return;
       case 6: gemv_run_fixed<6, DEPTH, DMA>(g, lane, acc); return;
+      case 7: gemv_run_fixed<7, DEPTH, DMA>(g, lane, acc); return;
       case 8:
         // two tables: eight straight-line steps exceed the register budget
         if constexpr (TABLES == 1) {
@@ -1287,6 +1294,7 @@ void decode_down_multi_kernel(const DecodeArgs a) {
     if (lane == 0 && any) a.valid[0] = 0;
   }
 }
+
 }  // namespace
 
 bool decode_path_fits(int64_t hidden, int64_t intermediate) {

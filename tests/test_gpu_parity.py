@@ -555,6 +555,27 @@ def test_routed_experts_matches_oracle(device, tokens, experts, hidden, inter, t
     print(cfg, assert_moe_close(host_f32(out), ref))
 
 
+# The decode kernels' straight-line streams: 3, 5 and 7 steps of 256 a wave in
+# gate/up (H / 4 waves) and in down (I), single-token and multi kernels, and K
+# ranges whose last waves have fewer steps (H = 2304: 3, 3, 3, 0).
+@pytest.mark.parametrize("tokens", [1, 3])
+@pytest.mark.parametrize("hidden,inter", [(3072, 768), (5120, 1280), (7168, 1792), (2304, 512)])
+def test_decode_step_counts_match_oracle(device, tokens, hidden, inter):
+    from glm_moe.layers.moe.routed_experts import routed_experts
+
+    cfg, x, ids, w, tables = _small_case(tokens, 4, hidden, inter, 2, 0.0, seed=hidden + tokens)
+    t = _device_tables(tables, device)
+    out, ok = routed_experts(bf16_dev(x, device), dev(ids, device), dev(w, device), *(t[k] for k in TABLE_KEYS))
+    ref, ref_ok = O.routed_experts(x, ids, w, **tables)
+    assert bool(ok) and ref_ok
+    # rows of up to 7168 N(0, 1) values give route rows larger than their sum: a
+    # flip is one bf16 ulp of a route's down row, which its weight (below 1)
+    # leaves at most two ulps of the weighted row
+    rows = [O.routed_experts(x, ids, np.where(np.arange(2) == s, w, 0).astype(np.float32), **tables)[0]
+            for s in range(2)]
+    print(cfg, assert_moe_close(host_f32(out), ref, flip_ulps=2.0, magnitude=np.maximum(*np.abs(rows))))
+
+
 # Stripe runs: an FP8 prefill work item of the down projection on 256-row
 # stripes runs up to 4 weight stripes of one tile in one continuous ring when K
 # has at least 4 blocks.  H = 1280 gives 5 such stripes (a run of 4, then a
