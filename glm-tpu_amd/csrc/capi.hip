@@ -884,6 +884,14 @@ int glm_moe_routed_projection(const uint16_t* lhs, int32_t slots, int64_t k, int
     return fail(GLM_MOE_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given",
                 glm_moe_routed_projection_workspace_bytes(slots), workspace_bytes);
   hipStream_t s = as_stream(stream);
+  if (routed_projection_fits(n, k)) {
+    const uint8_t* const bits[2] = {bits0, bits1};
+    const float* const scale[2] = {scale0, scale1};
+    GLM_HIP(launch_routed_projection(lhs, slots, (int32_t)k, tables, bits, scale, experts, (int32_t)n,
+                                     local_expert_ids, owned, result_dtype == GLM_MOE_F32, out, s),
+            "routed projection launch");
+    return GLM_MOE_OK;
+  }
   int32_t* tile_expert = static_cast<int32_t*>(workspace);
   int32_t* tile_row = tile_expert + slots;
   int32_t* tile_live = tile_row + slots;

@@ -1295,6 +1295,110 @@ void decode_down_multi_kernel(const DecodeArgs a) {
   }
 }
 
+// ------------------------------------------------------------------ the routed projection by itself
+// fp8_routed_projection: one row per slot against its expert in TABLES tables.
+// Workgroup = (slot, 16 weight rows of every table), four waves splitting K,
+// as the gate/up kernels: bound by HBM, whose stream the vector ALU keeps up
+// with where MFMA tiles of one live row in four did not (8 slots, two tables of
+// 2048 x 6144: 39 us after launches of 4 and 3 us for zeroed outputs and a slot
+// list; now one launch, the whole call 45.1 -> 31.8 us; 64 slots 265 -> 219).  Two owned slots of one
+// expert (of 64 consecutive slots) share a workgroup, which streams and
+// decodes the expert's rows once; an unowned slot's workgroups write zeros.
+struct ProjectionArgs {
+  const uint16_t* x;       // [slots, k] bf16
+  const uint8_t* bits[2];
+  const float* scale[2];
+  const int32_t* ids;
+  const uint8_t* owned;
+  int32_t slots, experts, n, k;
+  int32_t f32;
+  void* out;               // [slots, TABLES, n] f32 or bf16
+};
+
+template <int TABLES>
+__device__ __forceinline__ void projection_store(const ProjectionArgs& a, int slot, int t, int row, float v) {
+  const int64_t o = ((int64_t)slot * TABLES + t) * a.n + row;
+  if (a.f32)
+    static_cast<float*>(a.out)[o] = v;
+  else
+    static_cast<uint16_t*>(a.out)[o] = f32_to_bf16_bits(v);
+}
+
+template <int TABLES, int WK, int NR>
+__device__ __forceinline__ void projection_rows(const ProjectionArgs& a, int expert, const int (&slot)[NR],
+                                                int wave_steps, int wk, int lane, uint8_t* smem) {
+  float(*red)[2][TABLES][kGemvRows] = reinterpret_cast<float(*)[2][TABLES][kGemvRows]>(smem);
+  const int row0 = blockIdx.y * kGemvRows;
+  const int steps = (a.k + kStepK - 1) / kStepK;
+  GemvStream<TABLES, NR> g;
+  g.k = a.k;
+  g.kblocks = a.k / kScaleBlock;
+  g.row_stride = a.k;
+  g.lane_off = (uint32_t)((lane >> 4) * a.k + (lane & 15) * 16);
+  g.step_begin = min(wk * wave_steps, steps);
+  g.step_end = min(g.step_begin + wave_steps, steps);
+#pragma unroll
+  for (int t = 0; t < TABLES; ++t) {
+    g.w[t] = rows_buffer(a.bits[t] + ((int64_t)expert * a.n + row0) * a.k, (int64_t)kGemvRows * a.k);
+    const float* srow = a.scale[t] + ((int64_t)expert * (a.n / kScaleBlock) + row0 / kScaleBlock) * g.kblocks;
+    g.sreg[t] = lane_scale(srow, g.kblocks, g.step_begin, lane);
+  }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) g.x[r] = a.x + (int64_t)slot[r] * a.k;
+  g.xs_stride = xs_elems(wave_steps);
+  g.xs = reinterpret_cast<uint16_t*>(smem + sizeof(float) * WK * 2 * TABLES * kGemvRows) + wk * 2 * g.xs_stride;
+  g.pad = wave_steps * kStepK;
+  float acc[TABLES][4][NR] = {};
+  gemv_run<TABLES == 2 ? kGateUpDepth : 2 * kGateUpDepth, (NR > 1)>(g, lane, acc);
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+#pragma unroll
+    for (int t = 0; t < TABLES; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v = sum16(acc[t][q][r]);
+        if ((lane & 15) == 0) red[wk][r][t][4 * q + (lane >> 4)] = v;
+      }
+  __syncthreads();
+  // one thread per (slot, table, row): the waves' K ranges in wave order
+  const int tid = threadIdx.x;
+  if (tid < NR * TABLES * kGemvRows) {
+    const int row = tid % kGemvRows, t = tid / kGemvRows % TABLES, r = tid / (kGemvRows * TABLES);
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < WK; ++w) v += red[w][r][t][row];
+    projection_store<TABLES>(a, r == 0 ? slot[0] : slot[NR - 1], t, row0 + row, v);
+  }
+}
+
+template <int TABLES, int WK>
+__global__ __launch_bounds__(64 * WK) __attribute__((amdgpu_waves_per_eu(4)))
+void routed_projection_kernel(const ProjectionArgs a, int wave_steps) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int lane = threadIdx.x & 63;
+  const int wk = uniform(threadIdx.x >> 6);
+  const int slot = blockIdx.x, base = slot & ~63, own = slot & 63;
+  const int s = base + lane;
+  const int key = s < a.slots && a.owned[s] != 0 ? min(max(a.ids[s], 0), a.experts - 1) : -1;
+  const int expert = __builtin_amdgcn_readlane(key, own);
+  if (expert < 0) {
+    const int tid = threadIdx.x;
+    if (tid < TABLES * kGemvRows)
+      projection_store<TABLES>(a, slot, tid / kGemvRows, blockIdx.y * kGemvRows + tid % kGemvRows, 0.0f);
+    return;
+  }
+  const uint64_t same = __ballot(key == expert);
+  if (__popcll(same & ((1ull << own) - 1)) & 1) return;  // the second of a pair: the first's workgroup computes it
+  const uint64_t rest = same & ~((2ull << own) - 1);     // own = 63: none
+  if (rest != 0) {
+    const int pair[2] = {slot, base + uniform(__ffsll((unsigned long long)rest) - 1)};
+    projection_rows<TABLES, WK, 2>(a, expert, pair, wave_steps, wk, lane, smem);
+  } else {
+    const int one[1] = {slot};
+    projection_rows<TABLES, WK, 1>(a, expert, one, wave_steps, wk, lane, smem);
+  }
+}
+
 }  // namespace
 
 bool decode_path_fits(int64_t hidden, int64_t intermediate) {
@@ -1360,6 +1464,44 @@ hipError_t launch_decode_multi(const DecodeArgs& a, hipStream_t stream, const La
                          dim3(64 * kDownMultiWaves), d_lds, stream, a);
   return launch_kernel(decode_down_multi_kernel<kDownMultiWaves, false>, dim3(a.hidden / kDownRows),
                        dim3(64 * kDownMultiWaves), d_lds, stream, a);
+}
+
+bool routed_projection_fits(int64_t n, int64_t k) {
+  // a wave's quarter of K is staged in LDS (at most 2048), the weight rows of a
+  // workgroup go by blockIdx.y
+  return k % kScaleBlock == 0 && n % kScaleBlock == 0 && k <= kGateUpWaves * kMaxWaveSteps * kStepK &&
+         n / kGemvRows <= 65535;
+}
+
+hipError_t launch_routed_projection(const uint16_t* x, int32_t slots, int32_t k, int32_t tables,
+                                    const uint8_t* const* bits, const float* const* scale, int32_t experts, int32_t n,
+                                    const int32_t* ids, const uint8_t* owned, bool f32, void* out,
+                                    hipStream_t stream) {
+  if (slots <= 0 || experts <= 0 || tables < 1 || tables > 2 || !routed_projection_fits(n, k))
+    return hipErrorInvalidValue;
+  ProjectionArgs a{};
+  a.x = x;
+  for (int t = 0; t < tables; ++t) {
+    a.bits[t] = bits[t];
+    a.scale[t] = scale[t];
+  }
+  a.ids = ids;
+  a.owned = owned;
+  a.slots = slots;
+  a.experts = experts;
+  a.n = n;
+  a.k = k;
+  a.f32 = f32 ? 1 : 0;
+  a.out = out;
+  const int steps = gate_up_wave_steps(k);
+  const size_t lds = sizeof(float) * kGateUpWaves * 2 * tables * kGemvRows +
+                     sizeof(uint16_t) * kGateUpWaves * 2 * xs_elems(steps);
+  const dim3 grid(slots, n / kGemvRows);
+  label_next_launch("fp8_routed_projection_s%d_t%d_k%d_n%d_tn%d_tk%d", slots, tables, k, n, kGemvRows, kStepK);
+  return tables == 2 ? launch_kernel(routed_projection_kernel<2, kGateUpWaves>, grid, dim3(64 * kGateUpWaves), lds,
+                                     stream, a, steps)
+                     : launch_kernel(routed_projection_kernel<1, kGateUpWaves>, grid, dim3(64 * kGateUpWaves), lds,
+                                     stream, a, steps);
 }
 
 hipError_t launch_decode_routed(const DecodeArgs& a, hipStream_t stream, const LaunchEvents* stage_events) {

@@ -363,6 +363,15 @@ bool decode_path_fits(int64_t hidden, int64_t intermediate);
 // stage_events: null, or the armed events of the gate/up [0] and down [1] kernels.
 hipError_t launch_decode_routed(const DecodeArgs& a, hipStream_t stream, const LaunchEvents* stage_events);
 
+// The routed projection by itself (the reference's fp8_routed_projection): one
+// bf16 row per slot against its expert (ids clipped) in `tables` tables, out
+// [slots, tables, n] f32 or bf16, unowned slots zero; one launch.
+bool routed_projection_fits(int64_t n, int64_t k);
+hipError_t launch_routed_projection(const uint16_t* x, int32_t slots, int32_t k, int32_t tables,
+                                    const uint8_t* const* bits, const float* const* scale, int32_t experts, int32_t n,
+                                    const int32_t* ids, const uint8_t* owned, bool f32, void* out,
+                                    hipStream_t stream);
+
 // The bf16 shared expert over a few rows (tokens <= kSharedRowsMax): gate/up
 // [I, H], SwiGLU and down [H, I] with the resident path's rounding points,
 // every weight byte read once for all rows.  act: workspace [tokens, I] bf16.

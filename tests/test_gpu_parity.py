@@ -363,6 +363,37 @@ def test_routed_projection_matches_oracle(device, tables, dtype):
         np.testing.assert_allclose(actual, ref, rtol=2**-7, atol=2**-9)
 
 
+# The projection's kernel: one slot, pairs and odd rests of one expert's slots,
+# unowned slots between them, 64 and more slots (pairs form within 64), one K
+# block, an odd count of K blocks, the largest K it takes (8192) and one past it
+# (the grouped tiles).
+@pytest.mark.parametrize("slots,experts,n,k,tables", [
+    (1, 3, 128, 128, 1), (7, 2, 256, 640, 2), (64, 5, 128, 256, 1), (131, 3, 128, 384, 2), (5, 4, 256, 8192, 2),
+    (3, 2, 128, 8320, 1),
+])
+def test_routed_projection_slots_match_oracle(device, slots, experts, n, k, tables):
+    from glm_moe.kernels.fp8_grouped_matmul.kernel import RoutedProjectionConfig, fp8_routed_projection
+
+    rng = np.random.default_rng(slots + k)
+    x = O.bf16_round(rng.normal(0, 0.2, (slots, k)).astype(np.float32))
+    pairs = []
+    for _ in range(tables):
+        bits = torch.from_numpy(rng.normal(0, 0.15, (experts, n, k)).astype(np.float32)).to(
+            torch.float8_e4m3fn).view(torch.uint8).numpy()
+        pairs.append((bits, rng.uniform(0.1, 2.0, (experts, n // 128, k // 128)).astype(np.float32)))
+    ids = rng.integers(-2, experts + 2, slots).astype(np.int32)
+    owned = rng.random(slots) < 0.8
+    owned[0] = True
+    got = fp8_routed_projection(
+        bf16_dev(x, device), tuple((dev(b, device), dev(s, device)) for b, s in pairs), dev(ids, device),
+        dev(owned, device), config=RoutedProjectionConfig(output_tile=128, contraction_tile=128))
+    ref = O.routed_projection(x, tuple(pairs), ids, owned, result_dtype="float32")
+    actual = host_f32(got)
+    np.testing.assert_array_equal(actual[~owned], 0)
+    # FP32 sums of K exact products in another order (as the panel tiles' bound)
+    np.testing.assert_allclose(actual, ref, rtol=1e-5, atol=8 * 2**-24 * np.sqrt(k) * np.abs(ref).max())
+
+
 # ----------------------------------------------------------------------------- routed experts
 @pytest.fixture(scope="module")
 def golden():
