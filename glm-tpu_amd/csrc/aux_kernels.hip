@@ -66,6 +66,32 @@ __global__ void gather_rows_kernel(const uint32_t* src, int64_t src_rows, int64_
   }
 }
 
+// The same on 16-byte-aligned rows of a multiple of 16 bytes: `lanes` threads
+// (a power of two up to 256) share a row, look its index up once and move it in
+// 16-byte pieces, four in flight a thread.  Bound by HBM and the L2; the dword
+// kernel above spent its time on an index lookup and a division per dword (4000
+// rows of 12 KB: 35.6 us, here 16.8).
+__global__ __launch_bounds__(256) void gather_rows_x16_kernel(const u32x4* src, int64_t src_rows, int row_pieces,
+                                                              const int32_t* index, int32_t div,
+                                                              const uint8_t* mask, int64_t n, u32x4* dst, int lanes) {
+  const int64_t row = (int64_t)blockIdx.x * (blockDim.x / lanes) + threadIdx.x / lanes;
+  if (row >= n) return;
+  const bool keep = mask == nullptr || mask[row] != 0;
+  int64_t s = keep ? index[row] / div : 0;
+  s = s < 0 ? 0 : (s >= src_rows ? src_rows - 1 : s);
+  const u32x4* const from = src + s * row_pieces;
+  u32x4* const to = dst + row * row_pieces;
+  for (int w = threadIdx.x % lanes; w < row_pieces; w += 4 * lanes) {
+    u32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      v[j] = keep && w + j * lanes < row_pieces ? from[w + j * lanes] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (w + j * lanes < row_pieces) to[w + j * lanes] = v[j];
+  }
+}
+
 // pack_expert_panel_rows (panels.py:86-95): [capacity, panel_rows, row] with
 // rows beyond a panel's live count zero.
 __global__ void pack_panel_rows_kernel(const uint32_t* src, int64_t src_rows, int64_t row_words,
@@ -477,6 +503,17 @@ hipError_t launch_gather_rows(const void* src, int64_t src_rows, int64_t row_byt
   const int64_t words = row_bytes / 4;
   if (n * words == 0) return hipSuccess;
   label_next_launch("gather_prefill_route_rows_r%lld_b%lld", (long long)n, (long long)row_bytes);
+  if (row_bytes % 16 == 0 && row_bytes / 16 <= INT32_MAX / 2 &&
+      ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0) {
+    const int pieces = (int)(row_bytes / 16);
+    int lanes = 1;
+    while (lanes < 256 && 2 * lanes < pieces) lanes *= 2;  // two pieces a thread of a short row
+    const int64_t blocks = (n + 256 / lanes - 1) / (256 / lanes);
+    if (blocks <= INT32_MAX)
+      return launch_kernel(gather_rows_x16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
+                           static_cast<const u32x4*>(src), src_rows, pieces, index, div, mask, n,
+                           static_cast<u32x4*>(dst), lanes);
+  }
   return launch_kernel(gather_rows_kernel, grid_for(n * words, 256), dim3(256), 0, stream,
                      static_cast<const uint32_t*>(src), src_rows, words, index, div, mask, n,
                      static_cast<uint32_t*>(dst));

@@ -210,6 +210,27 @@ def test_build_expert_panels_edge_cases_are_bit_exact(device, counts, offset):
     _panels_equal(got, O.build_expert_panels(c, offset, rows=rows, local_groups=local))
 
 
+# Gathered rows: dword rows, one 16-byte piece, pieces that are no power of two,
+# rows past one pass of a workgroup's threads; clamped indexes, masked rows, and
+# a source that is only dword-aligned.
+@pytest.mark.parametrize("words", [3, 4, 12, 20, 260, 1028, 4100])
+@pytest.mark.parametrize("rows,offset", [(1, 0), (37, 0), (37, 1)])
+def test_gather_rows_is_bit_exact(device, words, rows, offset):
+    from glm_moe import _lib
+
+    g = torch.Generator(device=device).manual_seed(words)
+    flat = torch.randint(-2**31, 2**31 - 1, (23 * words + offset,), generator=g, device=device, dtype=torch.int64)
+    src = flat.to(torch.int32)[offset:].view(23, words)
+    index = torch.randint(-9, 3 * 26, (rows,), generator=g, device=device, dtype=torch.int32)
+    mask = torch.rand(rows, generator=g, device=device) < 0.7
+    for m in (None, mask):
+        dst = torch.empty((rows, words), dtype=torch.int32, device=device)
+        _lib.call("glm_moe_gather_rows", _lib.ptr(src), 23, words * 4, _lib.ptr(index), 3, _lib.ptr(m), rows,
+                  _lib.ptr(dst), _lib.stream_of(dst))
+        want = src[(index.double() / 3).trunc().long().clamp(0, 22)]  # C division truncates
+        assert torch.equal(dst, want if m is None else want * m[:, None])
+
+
 # ----------------------------------------------------------------------------- panel matmul
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_panel_matmul_matches_oracle(device, dtype):
