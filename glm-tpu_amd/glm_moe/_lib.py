@@ -8,8 +8,11 @@ already live on the GPU.
 from __future__ import annotations
 
 import ctypes
+import functools
 import re
 from pathlib import Path
+
+import torch
 
 LIB_PATH = Path(__file__).resolve().with_name("libglm_moe.so")
 HEADER_PATH = Path(__file__).resolve().parents[2] / "include" / "glm_moe.h"
@@ -159,21 +162,20 @@ def check(status: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    status = getattr(_LIB or lib(), name)(*args)
+    if status:
+        check(status)
 
 
-def ptr(tensor) -> ctypes.c_void_p:
-    """Device pointer of a tensor (None -> NULL)."""
-    if tensor is None:
-        return ctypes.c_void_p(0)
-    return ctypes.c_void_p(tensor.data_ptr())
+def ptr(tensor) -> int | None:
+    """Device pointer of a tensor (None -> NULL), as the c_void_p arguments take it."""
+    return None if tensor is None else tensor.data_ptr()
 
 
-def stream_of(tensor) -> ctypes.c_void_p:
-    """The current torch stream of the tensor's device as a hipStream_t."""
-    import torch
-
-    return ctypes.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
+def stream_of(tensor) -> int:
+    """The current torch stream of the tensor's device as a hipStream_t (read per
+    call, without the Stream object torch.cuda.current_stream builds: 1.5 us)."""
+    return torch._C._cuda_getCurrentRawStream(tensor.get_device())
 
 
 def require_device(*tensors) -> None:
@@ -185,8 +187,15 @@ def require_device(*tensors) -> None:
         if not t.is_cuda:
             raise ValueError("glm_moe kernels take GPU tensors only (no CPU fallback)")
         if device is None:
-            device = t.device
-        elif t.device != device:
+            device = t.get_device()
+        elif t.get_device() != device:
             raise ValueError("glm_moe tensors must share one device")
         if not t.is_contiguous():
             raise ValueError("glm_moe tensors must be contiguous")
+
+
+@functools.lru_cache(maxsize=1024)
+def size_query(name: str, *sizes: int) -> int:
+    """A host-only query of the library that depends on sizes alone (workspace
+    bytes, which kernels a geometry runs on)."""
+    return int(getattr(lib(), name)(*sizes))

@@ -111,8 +111,8 @@ def fp8_routed_projection(
     _lib.require_device(*tensors)
     tables = len(weights)
     out = torch.empty((slots, tables, output), dtype=result_dtype, device=lhs.device)
-    workspace = torch.empty(_lib.lib().glm_moe_routed_projection_workspace_bytes(slots), dtype=torch.uint8,
-                            device=lhs.device)
+    workspace = torch.empty(_lib.size_query("glm_moe_routed_projection_workspace_bytes", slots),
+                            dtype=torch.uint8, device=lhs.device)
     bits1, scale1 = weights[1] if tables == 2 else (None, None)
     _lib.call(
         "glm_moe_routed_projection",

@@ -56,7 +56,7 @@ def prefill_panel_fp8_matmul(
         raise ValueError("panel FP8 geometry/dtypes disagree with M32/N256/K128")
     _lib.require_device(lhs, weight_bits, scale, panels.expert_ids, panels.row_starts, panels.live_counts)
     out = torch.empty((m, n), dtype=dtype, device=lhs.device)
-    nbytes = _lib.lib().glm_moe_panel_fp8_matmul_workspace_bytes(m, k, groups, n)
+    nbytes = _lib.size_query("glm_moe_panel_fp8_matmul_workspace_bytes", m, k, groups, n)
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=lhs.device) if nbytes else None
     _lib.call(
         "glm_moe_panel_fp8_matmul_ws",

@@ -66,7 +66,7 @@ def group_prefill_routes(route_indices: torch.Tensor, *, num_experts: int = 256)
     inverse = torch.empty(n, dtype=torch.int32, device=device)
     counts = torch.empty(num_experts, dtype=torch.int32, device=device)
     valid = torch.empty((), dtype=torch.bool, device=device)
-    scratch_bytes = int(_lib.lib().glm_moe_group_routes_workspace_bytes(tokens, top_k, num_experts))
+    scratch_bytes = _lib.size_query("glm_moe_group_routes_workspace_bytes", tokens, top_k, num_experts)
     scratch = torch.empty(max(scratch_bytes, 1), dtype=torch.uint8, device=device)
     _lib.call(
         "glm_moe_group_routes",
@@ -178,9 +178,9 @@ _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 def routed_workspace(tokens: int, top_k: int, num_experts: int, hidden: int, intermediate: int,
                      device: torch.device) -> torch.Tensor:
     """The workspace of ``routed_experts`` for a call on the current stream of
-    ``device``: a slice of that stream's buffer, grown when a call needs more."""
-    nbytes = max(int(_lib.lib().glm_moe_routed_experts_workspace_bytes(
-        tokens, top_k, num_experts, hidden, intermediate)), 1)
+    ``device``: that stream's buffer, grown when a call needs more."""
+    nbytes = max(_lib.size_query("glm_moe_routed_experts_workspace_bytes", tokens, top_k, num_experts, hidden,
+                                 intermediate), 1)
     device = torch.device(device)
     if torch.cuda.is_current_stream_capturing() or nbytes > WORKSPACE_CACHE_MAX:
         # under HIP graph capture: a buffer of the graph's private memory pool,
@@ -189,15 +189,15 @@ def routed_workspace(tokens: int, top_k: int, num_experts: int, hidden: int, int
         # torch's allocator, which reuses the block only for later work on this
         # stream once the caller drops it
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    stream = torch.cuda.current_stream(device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream.cuda_stream)
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    key = (index, torch._C._cuda_getCurrentRawStream(index))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:
         # the old buffer returns to torch's allocator in the order of its stream
         _WORKSPACES.pop(key, None)
         ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         _WORKSPACES[key] = ws
-    return ws[:nbytes]
+    return ws
 
 
 def release_workspaces() -> None:
@@ -255,24 +255,24 @@ def routed_experts(
     if route_indices.ndim != 2 or route_indices.shape[0] != tokens or route_indices.dtype != torch.int32:
         raise ValueError("route indices must be int32 [tokens, top_k]")
     top_k = route_indices.shape[1]
-    if tuple(route_weights.shape) != (tokens, top_k) or route_weights.dtype != torch.float32:
+    if route_weights.shape != (tokens, top_k) or route_weights.dtype != torch.float32:
         raise ValueError("route weights must be float32 [tokens, top_k]")
     if gate_bits.ndim != 3 or gate_bits.dtype != torch.uint8:
         raise ValueError("expert gate bits must be uint8 [E, I, H]")
     experts, inter, gh = gate_bits.shape
-    if gh != h or tuple(up_bits.shape) != (experts, inter, h) or tuple(down_bits.shape) != (experts, h, inter):
+    if gh != h or up_bits.shape != (experts, inter, h) or down_bits.shape != (experts, h, inter):
         raise ValueError("expert table geometry disagrees with the hidden size")
     if up_bits.dtype != torch.uint8 or down_bits.dtype != torch.uint8:
         raise ValueError("expert tables must be uint8 e4m3fn bits")
     for scale, rows, cols in ((gate_scale, inter, h), (up_scale, inter, h), (down_scale, h, inter)):
-        if scale.dtype != torch.float32 or tuple(scale.shape) != (experts, rows // 128, cols // 128):
+        if scale.dtype != torch.float32 or scale.shape != (experts, rows // 128, cols // 128):
             raise ValueError("expert scales must be float32 [E, N/128, K/128]")
     if route_sum not in ("float32", "bfloat16"):
         raise ValueError("route_sum must be float32 or bfloat16")
     if activations not in ("bfloat16", "float8_e4m3fn"):
         raise ValueError("activations must be bfloat16 or float8_e4m3fn")
     if shared is not None:
-        if tuple(shared.shape) != (tokens, h) or shared.dtype != torch.bfloat16 or not shared.is_contiguous():
+        if shared.shape != (tokens, h) or shared.dtype != torch.bfloat16 or not shared.is_contiguous():
             raise ValueError("shared expert rows must be contiguous bf16 [tokens, hidden]")
         if events is not None:
             raise ValueError("stage events time the routed experts alone")
@@ -284,9 +284,9 @@ def routed_experts(
         if (
             len(shared_tables) != 3
             or any(t.dtype != torch.bfloat16 or not t.is_contiguous() for t in shared_tables)
-            or tuple(shared_tables[0].shape) != (inter, h)
-            or tuple(shared_tables[1].shape) != (inter, h)
-            or tuple(shared_tables[2].shape) != (h, inter)
+            or shared_tables[0].shape != (inter, h)
+            or shared_tables[1].shape != (inter, h)
+            or shared_tables[2].shape != (h, inter)
         ):
             raise ValueError("resident shared expert tables must be contiguous bf16 [I, H], [I, H], [H, I]")
     _lib.require_device(hidden, route_indices, route_weights, gate_bits, gate_scale, up_bits, up_scale,
@@ -294,7 +294,7 @@ def routed_experts(
     device = hidden.device
     if out is None:
         out = torch.empty((tokens, h), dtype=torch.bfloat16, device=device)
-    elif tuple(out.shape) != (tokens, h) or out.dtype != torch.bfloat16:
+    elif out.shape != (tokens, h) or out.dtype != torch.bfloat16:
         raise ValueError("out must be bf16 [tokens, hidden]")
     valid = torch.empty((), dtype=torch.bool, device=device)
     ws = routed_workspace(tokens, top_k, experts, h, inter, device)
@@ -362,20 +362,20 @@ def routed_experts_from_router_logits(
     if gate_bits.ndim != 3 or gate_bits.dtype != torch.uint8:
         raise ValueError("expert gate bits must be uint8 [E, I, H]")
     experts, inter, gh = gate_bits.shape
-    if gh != h or tuple(up_bits.shape) != (experts, inter, h) or tuple(down_bits.shape) != (experts, h, inter):
+    if gh != h or up_bits.shape != (experts, inter, h) or down_bits.shape != (experts, h, inter):
         raise ValueError("expert table geometry disagrees with the hidden size")
     for scale, rows, cols in ((gate_scale, inter, h), (up_scale, inter, h), (down_scale, h, inter)):
-        if scale.dtype != torch.float32 or tuple(scale.shape) != (experts, rows // 128, cols // 128):
+        if scale.dtype != torch.float32 or scale.shape != (experts, rows // 128, cols // 128):
             raise ValueError("expert scales must be float32 [E, N/128, K/128]")
-    if router_logits.ndim != 2 or tuple(router_logits.shape) != (tokens, experts):
+    if router_logits.ndim != 2 or router_logits.shape != (tokens, experts):
         raise ValueError(f"router_logits must have shape {(tokens, experts)}")
-    if correction_bias is not None and tuple(correction_bias.shape) != (experts,):
+    if correction_bias is not None and correction_bias.shape != (experts,):
         raise ValueError(f"correction_bias must have shape {(experts,)}")
     if not isinstance(top_k, int) or isinstance(top_k, bool) or not 0 < top_k <= min(experts, 64):
         raise ValueError("top_k must be in [1, min(num_experts, 64)]")
     if route_sum not in ("float32", "bfloat16") or activations not in ("bfloat16", "float8_e4m3fn"):
         raise ValueError("route_sum must be float32 or bfloat16; activations bfloat16 or float8_e4m3fn")
-    if shared is not None and (tuple(shared.shape) != (tokens, h) or shared.dtype != torch.bfloat16
+    if shared is not None and (shared.shape != (tokens, h) or shared.dtype != torch.bfloat16
                                or not shared.is_contiguous()):
         raise ValueError("shared expert rows must be contiguous bf16 [tokens, hidden]")
     _lib.require_device(hidden, router_logits, correction_bias, gate_bits, gate_scale, up_bits, up_scale,
@@ -385,7 +385,7 @@ def routed_experts_from_router_logits(
     bias = None if correction_bias is None else correction_bias.float().contiguous()
     if out is None:
         out = torch.empty((tokens, h), dtype=torch.bfloat16, device=device)
-    elif tuple(out.shape) != (tokens, h) or out.dtype != torch.bfloat16:
+    elif out.shape != (tokens, h) or out.dtype != torch.bfloat16:
         raise ValueError("out must be bf16 [tokens, hidden]")
     ids = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
     weights = torch.empty((tokens, top_k), dtype=torch.float32, device=device)
@@ -437,15 +437,15 @@ def routed_experts_share(
     if route_indices.ndim != 2 or route_indices.shape[0] != tokens or route_indices.dtype != torch.int32:
         raise ValueError("route indices must be int32 [tokens, top_k]")
     top_k = route_indices.shape[1]
-    if tuple(route_weights.shape) != (tokens, top_k) or route_weights.dtype != torch.float32:
+    if route_weights.shape != (tokens, top_k) or route_weights.dtype != torch.float32:
         raise ValueError("route weights must be float32 [tokens, top_k]")
     if gate_bits.ndim != 3 or gate_bits.dtype != torch.uint8:
         raise ValueError("expert gate bits must be uint8 [E_local, I, H]")
     local, inter, gh = gate_bits.shape
-    if gh != h or tuple(up_bits.shape) != (local, inter, h) or tuple(down_bits.shape) != (local, h, inter):
+    if gh != h or up_bits.shape != (local, inter, h) or down_bits.shape != (local, h, inter):
         raise ValueError("expert table geometry disagrees with the hidden size")
     for scale, rows, cols in ((gate_scale, inter, h), (up_scale, inter, h), (down_scale, h, inter)):
-        if scale.dtype != torch.float32 or tuple(scale.shape) != (local, rows // 128, cols // 128):
+        if scale.dtype != torch.float32 or scale.shape != (local, rows // 128, cols // 128):
             raise ValueError("expert scales must be float32 [E_local, N/128, K/128]")
     if not 0 <= expert_offset <= num_experts - local:
         raise ValueError(f"the share's experts [{expert_offset}, {expert_offset + local}) lie outside "
@@ -456,7 +456,7 @@ def routed_experts_share(
                         down_bits, down_scale, out)
     if out is None:
         out = torch.empty((tokens, h), dtype=torch.float32, device=hidden.device)
-    elif tuple(out.shape) != (tokens, h) or out.dtype != torch.float32:
+    elif out.shape != (tokens, h) or out.dtype != torch.float32:
         raise ValueError("out must be float32 [tokens, hidden]")
     valid = torch.empty((), dtype=torch.bool, device=hidden.device)
     ws = routed_workspace(tokens, top_k, local, h, inter, hidden.device)
@@ -478,7 +478,7 @@ def moe_layer_epilogue(routed: torch.Tensor, shared: torch.Tensor, valid: torch.
     non-finite output clears ``valid`` in place (``:126``)."""
     if routed.ndim != 2 or routed.dtype != torch.float32:
         raise ValueError("the routed sum must be float32 [tokens, hidden]")
-    if tuple(shared.shape) != tuple(routed.shape) or shared.dtype != torch.bfloat16:
+    if shared.shape != routed.shape or shared.dtype != torch.bfloat16:
         raise ValueError("shared expert rows must be bf16 [tokens, hidden]")
     if valid.dtype != torch.bool or valid.numel() != 1:
         raise ValueError("valid must be a one-element bool tensor")
@@ -505,7 +505,7 @@ def swiglu_bf16(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
 def uses_decode_kernels(tokens: int, top_k: int, hidden: int, intermediate: int) -> bool:
     """Whether a layer of this geometry runs on the two decode kernels (where the
     shared expert can run inside them)."""
-    return bool(_lib.lib().glm_moe_uses_decode_kernels(tokens, top_k, hidden, intermediate))
+    return bool(_lib.size_query("glm_moe_uses_decode_kernels", tokens, top_k, hidden, intermediate))
 
 
 def _shared_swiglu(hidden: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, down: torch.Tensor) -> torch.Tensor:
@@ -545,13 +545,13 @@ def shared_expert_rows(hidden: torch.Tensor, gate: torch.Tensor, up: torch.Tenso
     inter = gate.shape[0]
     if not shared_expert_rows_fit(tokens, h, inter):
         raise ValueError("the few-row shared expert takes 1..8 rows and sizes that are multiples of 128, <= 8192")
-    if (tuple(gate.shape) != (inter, h) or tuple(up.shape) != (inter, h) or tuple(down.shape) != (h, inter)
+    if (gate.shape != (inter, h) or up.shape != (inter, h) or down.shape != (h, inter)
             or any(t.dtype != torch.bfloat16 for t in (hidden, gate, up, down))):
         raise ValueError("shared expert tables must be bf16 [I, H], [I, H], [H, I] for bf16 [T, H] rows")
     x, g, u, d = (t.contiguous() for t in (hidden, gate, up, down))
     _lib.require_device(x, g, u, d)
     out = torch.empty((tokens, h), dtype=torch.bfloat16, device=x.device)
-    ws = torch.empty(int(_lib.lib().glm_moe_shared_expert_rows_workspace_bytes(tokens, inter)),
+    ws = torch.empty(_lib.size_query("glm_moe_shared_expert_rows_workspace_bytes", tokens, inter),
                      dtype=torch.uint8, device=x.device)
     _lib.call("glm_moe_shared_expert_rows", _lib.ptr(x), tokens, h, _lib.ptr(g), _lib.ptr(u), _lib.ptr(d), inter,
               _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
@@ -577,16 +577,16 @@ def _check_layer_shapes(hidden_local, route_indices, route_weights, gate_bits, u
         raise ValueError("MoE hidden size differs from contract")
     if route_indices is not None:
         expected = (hidden_local.shape[0], contract.top_k)
-        if tuple(route_indices.shape) != expected or tuple(route_weights.shape) != expected:
+        if route_indices.shape != expected or route_weights.shape != expected:
             raise ValueError("routing geometry differs from contract")
         if route_indices.dtype != torch.int32:
             raise ValueError("routes must be int32")
         if route_weights.dtype != torch.float32:
             raise ValueError("route weights must be FP32")
     gate_shape = (contract.local_experts, contract.intermediate_size, contract.hidden_size)
-    if tuple(gate_bits.shape) != gate_shape or tuple(up_bits.shape) != gate_shape:
+    if gate_bits.shape != gate_shape or up_bits.shape != gate_shape:
         raise ValueError("expert gate/up geometry differs from contract")
-    if tuple(down_bits.shape) != (contract.local_experts, contract.hidden_size, contract.intermediate_size):
+    if down_bits.shape != (contract.local_experts, contract.hidden_size, contract.intermediate_size):
         raise ValueError("expert down geometry differs from contract")
 
 
@@ -644,9 +644,9 @@ def prefill_moe_from_routes(
         raise ValueError("expert panels require checkpoint scale blocks128x128")
     inter, h = contract.intermediate_size, contract.hidden_size
     if (
-        tuple(shared_gate_local.shape) != (inter, h)
-        or tuple(shared_up_local.shape) != (inter, h)
-        or tuple(shared_down_local.shape) != (h, inter)
+        shared_gate_local.shape != (inter, h)
+        or shared_up_local.shape != (inter, h)
+        or shared_down_local.shape != (h, inter)
     ):
         raise ValueError("prefill shared expert geometry differs from contract")
     tables = (shared_gate_local, shared_up_local, shared_down_local)
@@ -708,7 +708,7 @@ def prefill_moe_from_router_logits(
     if contract.stage_size != 1:
         raise ValueError("routing inside the layer takes a one-GPU contract; for an expert-parallel share route "
                          "with route_glm_noaux_tc_logits and call prefill_moe_from_routes")
-    if router_logits.ndim != 2 or tuple(router_logits.shape) != (hidden_local.shape[0], contract.num_experts):
+    if router_logits.ndim != 2 or router_logits.shape != (hidden_local.shape[0], contract.num_experts):
         raise ValueError(f"router_logits must have shape {(hidden_local.shape[0], contract.num_experts)}")
     top_k = contract.top_k
     inter, h = contract.intermediate_size, contract.hidden_size
@@ -717,8 +717,8 @@ def prefill_moe_from_router_logits(
     if contract.fp8_block_shape != (128, 128):
         raise ValueError("expert panels require checkpoint scale blocks128x128")
     tables = (shared_gate_local, shared_up_local, shared_down_local)
-    if (tuple(tables[0].shape) != (inter, h) or tuple(tables[1].shape) != (inter, h)
-            or tuple(tables[2].shape) != (h, inter)):
+    if (tables[0].shape != (inter, h) or tables[1].shape != (inter, h)
+            or tables[2].shape != (h, inter)):
         raise ValueError("prefill shared expert geometry differs from contract")
     rows = hidden_local.shape[0]
     logits = router_logits.float().contiguous()
@@ -744,7 +744,7 @@ def prefill_moe_from_router_logits(
             *(_lib.ptr(t) for t in resident), inter, float(contract.routed_scaling_factor), _lib.ptr(ids),
             _lib.ptr(weights), _lib.ptr(out), _lib.ptr(layer_valid), _lib.ptr(ws), ws.numel(),
             _lib.stream_of(hidden_local))
-    elif decode and rows > 1 and correction_bias is not None and tuple(correction_bias.shape) == (
+    elif decode and rows > 1 and correction_bias is not None and correction_bias.shape == (
             contract.num_experts,):
         # a few rows: the router kernel, then the decode kernels with the resident
         # shared expert (its weights streamed once per group of up to 4 rows)
@@ -811,9 +811,9 @@ def moe_grouped_routes(
     if (
         len(shared_bf16) != 3
         or any(t.dtype != torch.bfloat16 for t in shared_bf16)
-        or tuple(shared_bf16[0].shape) != (inter, h)
-        or tuple(shared_bf16[1].shape) != (inter, h)
-        or tuple(shared_bf16[2].shape) != (h, inter)
+        or shared_bf16[0].shape != (inter, h)
+        or shared_bf16[1].shape != (inter, h)
+        or shared_bf16[2].shape != (h, inter)
     ):
         raise ValueError("grouped MoE BF16 shared tables drifted")
     if contract.stage_size > 1:
@@ -869,9 +869,9 @@ def moe_mlp_from_router_logits(
     from glm_moe.layers.moe.router import route_glm_noaux_tc_logits
 
     experts, top_k = contract.num_experts, contract.top_k  # the router scores every expert
-    if router_logits.ndim != 2 or tuple(router_logits.shape) != (hidden_local.shape[0], experts):
+    if router_logits.ndim != 2 or router_logits.shape != (hidden_local.shape[0], experts):
         raise ValueError(f"router_logits must have shape {(hidden_local.shape[0], experts)}")
-    if correction_bias is not None and tuple(correction_bias.shape) != (experts,):
+    if correction_bias is not None and correction_bias.shape != (experts,):
         raise ValueError(f"correction_bias must have shape {(experts,)}")
     inter, h = contract.intermediate_size, contract.hidden_size
     fused = (
@@ -894,14 +894,14 @@ def moe_mlp_from_router_logits(
     if (
         len(shared_bf16) != 3
         or any(t.dtype != torch.bfloat16 for t in shared_bf16)
-        or tuple(shared_bf16[0].shape) != (inter, h)
-        or tuple(shared_bf16[1].shape) != (inter, h)
-        or tuple(shared_bf16[2].shape) != (h, inter)
+        or shared_bf16[0].shape != (inter, h)
+        or shared_bf16[1].shape != (inter, h)
+        or shared_bf16[2].shape != (h, inter)
     ):
         raise ValueError("grouped MoE BF16 shared tables drifted")
     for scale, rows, cols in ((expert_gate_scale_local, inter, h), (expert_up_scale_local, inter, h),
                               (expert_down_scale_local, h, inter)):
-        if scale.dtype != torch.float32 or tuple(scale.shape) != (experts, rows // 128, cols // 128):
+        if scale.dtype != torch.float32 or scale.shape != (experts, rows // 128, cols // 128):
             raise ValueError("expert scales must be float32 [E, N/128, K/128]")
     tables = tuple(t.contiguous() for t in shared_bf16)
     logits = router_logits.float().contiguous()
