@@ -65,15 +65,18 @@ constexpr int kChunk = 32;         // work items dealt to an XCD together: one p
 
 // Work item of workgroup b (-1: none) when `total` items are dealt in chunks:
 // the q-th workgroup of XCD x = b % 8 runs item (j * 8 + x') * 32 + q % 32 with
-// j = q / 32 and x' = x for even j, 7 - x for odd j.  Each XCD runs `per`
-// workgroups, a whole number of chunks.
+// j = q / 32 and x' = x for even j, 7 - x for odd j, while whole rounds of 8
+// chunks last; the rest of the list is dealt in eighths, so that the launch ends
+// on every XCD's share of the HBM and not with 32 items on one.
 __device__ __forceinline__ int xcd_item(int b, int total) {
-  const int chunks = (total + kChunk - 1) / kChunk;
-  const int per = (chunks + kXcds - 1) / kXcds * kChunk;
-  const int q = b / kXcds;
-  if (q >= per) return -1;
-  const int j = q / kChunk, x = b % kXcds;
-  return (j * kXcds + ((j & 1) ? kXcds - 1 - x : x)) * kChunk + q % kChunk;
+  constexpr int kRound = kXcds * kChunk;
+  const int rounds = total / kRound, rest = total - rounds * kRound;
+  const int q = b / kXcds, x = b % kXcds;
+  const int j = q / kChunk, k = q % kChunk;
+  const int turn = (j & 1) ? kXcds - 1 - x : x;
+  if (j < rounds) return (j * kXcds + turn) * kChunk + k;
+  const int share = (rest + kXcds - 1) / kXcds, r = turn * share + k;
+  return j == rounds && k < share && r < rest ? rounds * kRound + r : -1;
 }
 // Stripes one work item runs: a.stripe_run, clamped to 1 .. kMaxStripeRun,
 // and 1 when K has fewer than kMinRunBlocks blocks (the rings look up to 3

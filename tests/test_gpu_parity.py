@@ -655,6 +655,38 @@ def test_prefill_stripe_runs_match_oracle(device, activations, hidden, inter, se
     print(cfg, activations, close(host_f32(out), ref))
 
 
+# Work items dealt to the XCDs: one item per expert in both projections (H 256, I
+# 128, every expert one route), around whole rounds of 256 items, eighths of the
+# rest, and more than one round.
+@pytest.mark.parametrize("experts", [65, 249, 255, 256, 257, 264, 265, 511, 520, 1000])
+def test_prefill_work_list_lengths_compute_every_item(device, experts):
+    from glm_moe.layers.moe.routed_experts import routed_experts
+
+    g = torch.Generator(device=device).manual_seed(experts)
+    x = torch.randn((experts, 256), generator=g, device=device).to(torch.bfloat16)
+    ids = torch.randperm(experts, generator=g, device=device).to(torch.int32)[:, None].contiguous()
+    w = torch.ones((experts, 1), device=device)
+
+    def table(n, k):
+        return (torch.randint(0, 120, (experts, n, k), generator=g, device=device, dtype=torch.int32).to(torch.uint8),
+                torch.rand((experts, n // 128, k // 128), generator=g, device=device) * 1e-3 + 1e-3)
+
+    tabs = [*table(128, 256), *table(128, 256), *table(256, 128)]
+    out, ok = routed_experts(x, ids, w, *tabs)
+    assert bool(ok)
+    dec = [(b[ids[:, 0].long()].view(torch.float8_e4m3fn).float()
+            * s[ids[:, 0].long()].repeat_interleave(128, 1).repeat_interleave(128, 2)).to(torch.bfloat16).double()
+           for b, s in zip(tabs[::2], tabs[1::2])]
+    gate, up = ((d * x.double()[:, None, :]).sum(2).to(torch.bfloat16).double() for d in dec[:2])
+    act = ((gate * torch.sigmoid(gate).to(torch.bfloat16).double()).to(torch.bfloat16).double() * up).to(
+        torch.bfloat16).double()
+    want = (dec[2] * act[:, None, :]).sum(2)
+    # a skipped item leaves rows of the workspace; a computed one is within bf16
+    # rounding of gate, up, the SwiGLU and the row (each 2**-9 of its value)
+    scale = (dec[2].abs() * act.abs()[:, None, :]).sum(2)
+    assert ((out.double() - want).abs() <= 2**-6 * scale).all()
+
+
 # Stripe geometries at their edges, both modes: tall down stripes with K = 1
 # block (I = 128, the two-slot ring's look-ahead past the end from the first
 # block on) beside 256-row gate/up stripes; tall gate/up with K = 2 blocks
