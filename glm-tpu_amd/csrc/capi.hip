@@ -272,6 +272,24 @@ struct RouterIn {
   const float* bias;
 };
 
+// The resident shared expert inside the prefill launches: its bf16 tables.
+struct SharedTables {
+  const uint16_t* gate;
+  const uint16_t* up;
+  const uint16_t* down;
+};
+// Its rows [tokens, H], behind the routed layout.
+size_t prefill_shared_bytes(int64_t tokens, int64_t hidden) {
+  return align_up(sizeof(uint16_t) * (size_t)tokens * (size_t)hidden);
+}
+// Whether a bf16 layer runs both projections on the pipelined prefill kernel.
+bool on_prefill_kernel(int64_t tokens, int32_t top_k, int32_t experts, int64_t hidden, int64_t intermediate) {
+  const int64_t n = tokens * top_k;
+  return !uses_decode_path(n, hidden, intermediate) &&
+         routed_shape(tokens, n, experts, hidden, intermediate) == kShapeWide && prefill_fits(intermediate, hidden, 2) &&
+         prefill_fits(hidden, intermediate, 1) && prefill_rows_fit(tokens, hidden) && prefill_rows_fit(n, intermediate);
+}
+
 int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_size,
                         const int32_t* route_indices, const float* route_weights, int32_t top_k,
                         int32_t num_experts, int64_t intermediate, const uint8_t* gate_bits,
@@ -281,7 +299,8 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
                         uint16_t* out, uint8_t* valid, void* workspace, size_t workspace_bytes,
                         const StageTimer& timer, void* stream_ptr, const RouterIn* router = nullptr,
                         bool compact_decode_scratch = false, int32_t global_experts = 0,
-                        int32_t expert_offset = 0, float* out_f32 = nullptr) {
+                        int32_t expert_offset = 0, float* out_f32 = nullptr,
+                        const SharedTables* shared_tables = nullptr) {
   // a whole layer unless the caller names a share: tables of num_experts experts
   // from global id expert_offset on, of global_experts in all
   if (global_experts == 0) global_experts = num_experts;
@@ -322,7 +341,11 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
   const RoutedLayout L = routed_layout(tokens, top_k, num_experts, hidden_size, intermediate);
   const bool decode = uses_decode_path(n, hidden_size, intermediate);
   GLM_REQUIRE(decode || !compact_decode_scratch, "the decode-path scratch layout takes decode shapes only");
-  const size_t need = compact_decode_scratch ? decode_scratch_bytes(tokens, top_k, intermediate) : L.total;
+  GLM_REQUIRE(shared_tables == nullptr ||
+                  (!fp8 && on_prefill_kernel(tokens, top_k, num_experts, hidden_size, intermediate)),
+              "the shared expert runs inside the bf16 prefill launches only");
+  const size_t need = (compact_decode_scratch ? decode_scratch_bytes(tokens, top_k, intermediate) : L.total) +
+                      (shared_tables != nullptr ? prefill_shared_bytes(tokens, hidden_size) : 0);
   if (workspace_bytes < need || workspace == nullptr)
     return fail(GLM_MOE_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given", need, workspace_bytes);
   hipStream_t stream = as_stream(stream_ptr);
@@ -504,6 +527,16 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
     g.outq = actq;
     g.outq_scale = actscale;
   }
+  uint16_t* const shared_act = reinterpret_cast<uint16_t*>(ws + L.act_shared);
+  uint16_t* const shared_rows = reinterpret_cast<uint16_t*>(ws + L.total);
+  if (shared_tables != nullptr) {
+    g.sw0 = shared_tables->gate;
+    g.sw1 = shared_tables->up;
+    g.sx = hidden;
+    g.sout = shared_act;
+    g.shared_rows = (int32_t)tokens;
+    g.shared_tiles = prefill_shared_tiles(tokens);
+  }
   timer.arm(kStageGateUp);
   GLM_HIP(launch_grouped_gemm(g, shape, 2, kEpiSwiglu, stream), "gate/up launch");
   timer.done(kStageGateUp);
@@ -543,6 +576,14 @@ int routed_experts_impl(const uint16_t* hidden, int64_t tokens, int64_t hidden_s
   d.tile_rows = tile_rows;
   d.wide_twice = p.wide_twice;
   d.tall = g.tall;
+  if (shared_tables != nullptr) {
+    d.sw0 = shared_tables->down;
+    d.sx = shared_act;
+    d.sout = shared_rows;
+    d.shared_rows = g.shared_rows;
+    d.shared_tiles = g.shared_tiles;
+    shared = shared_rows;
+  }
   timer.arm(kStageDown);
   GLM_HIP(launch_grouped_gemm(d, shape, 1, kEpiStoreBf16, stream), "down launch");
   timer.done(kStageDown);
@@ -1025,6 +1066,35 @@ int glm_moe_moe_layer_epilogue(const float* routed, int64_t tokens, int64_t hidd
                                 as_stream(stream)),
           "epilogue launch");
   return GLM_MOE_OK;
+}
+
+size_t glm_moe_moe_layer_shared_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t hidden,
+                                                int64_t intermediate) {
+  if (tokens <= 0 || top_k <= 0 || num_experts <= 0 || hidden <= 0 || intermediate <= 0 ||
+      tokens > INT32_MAX / 2 / top_k || !on_prefill_kernel(tokens, top_k, num_experts, hidden, intermediate))
+    return 0;
+  return routed_layout(tokens, top_k, num_experts, hidden, intermediate).total + prefill_shared_bytes(tokens, hidden);
+}
+
+int glm_moe_moe_layer_shared(const uint16_t* hidden, int64_t tokens, int64_t hidden_size,
+                             const float* router_logits, const float* correction_bias, int32_t* route_indices,
+                             float* route_weights, int32_t top_k, int32_t num_experts, int64_t intermediate,
+                             const uint8_t* gate_bits, const float* gate_scale, const uint8_t* up_bits,
+                             const float* up_scale, const uint8_t* down_bits, const float* down_scale, uint32_t flags,
+                             const uint16_t* shared_gate, const uint16_t* shared_up, const uint16_t* shared_down,
+                             float routed_scale, uint16_t* out, uint8_t* valid, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+  GLM_REQUIRE(shared_gate && shared_up && shared_down, "null shared expert table");
+  GLM_REQUIRE(std::isfinite(routed_scale), "routed scale must be finite");
+  GLM_REQUIRE(router_logits == nullptr || top_k <= kWave,
+              "the GPU router selects at most %d experts per token (one wave lane each)", kWave);
+  const SharedTables tables{shared_gate, shared_up, shared_down};
+  const RouterIn router{router_logits, correction_bias};
+  return routed_experts_impl(hidden, tokens, hidden_size, route_indices, route_weights, top_k, num_experts,
+                             intermediate, gate_bits, gate_scale, up_bits, up_scale, down_bits, down_scale, flags,
+                             nullptr, nullptr, bf16_round_host(routed_scale), out, valid, workspace, workspace_bytes,
+                             StageTimer{nullptr, nullptr}, stream, router_logits != nullptr ? &router : nullptr,
+                             false, 0, 0, nullptr, &tables);
 }
 
 int glm_moe_uses_decode_kernels(int64_t tokens, int32_t top_k, int64_t hidden_size, int64_t intermediate) {

@@ -424,6 +424,180 @@ constexpr int prefill_pending(int la, int sx, int xloads, int wloads) {
   return sx - 1 < la ? wloads + (sx - 2) * (xloads + wloads) : (la - 1) * (xloads + wloads);
 }
 
+// A work item of the resident shared expert in the same launch: 256 bf16
+// weight rows (128 of each of two tables) against up to 256 token rows, the
+// routed items' LDS rings and epilogue with bf16 weights as they are.  A row's
+// 128 bytes of a ring block are 64 K values, so a weight block goes with one
+// half-block activation stage, and nothing is decoded: MFMA steps 0 and 1 of
+// lane group g take chunks 2 g and 2 g + 1 of both operands' rows.  Loads, in
+// issue order: weight blocks 0 and 1, activations 0; then in block j the
+// activations of j + 1 (the stage freed by this block's barrier) and the
+// weights of j + 2 (the wave's own slot, read in block j - 1), so at a barrier
+// only a block's weight loads (WLOADS) may still be in flight.
+// Run by the launches of the routed projections because they are bound by
+// their weight stream (small prefills) or leave CUs idle at their ends, where
+// the shared expert as three GEMMs and a SwiGLU of its own (46 us at 61 rows,
+// 119 at 777, 190 at 2048) waits for them to finish: GLM-5-shape layer T=61
+// 1036 -> 1020 us, T=777 1708 -> 1674, T=2048 2229 -> 2190.
+template <int TABLES, int WAVES, int EPI, int NCG>
+__device__ __forceinline__ void shared_item_run(const GroupedGemmArgs& a, uint8_t* lds, int stripe, int r0, int live,
+                                                int wave, int lane) {
+  constexpr int GS = 2;                        // 16-row weight groups a wave
+  constexpr int RS = GS / TABLES;              // of each table
+  constexpr int BN = WAVES * RS * 16;
+  constexpr int SBLOCK = WAVES * GS * 2048;    // bytes of the item's weight rows per block
+  constexpr int SW = 3;
+  constexpr int WLOADS = GS * 2;
+  constexpr int XLOADS = (NCG * 2 + WAVES - 1) / WAVES;
+  constexpr int HSTAGE = XLOADS * WAVES * 1024;
+  static_assert(SBLOCK == kStripeBlockBytes && SW * SBLOCK + 2 * HSTAGE <= kPrefillLds, "LDS budget");
+  const int lrow = lane & 15, lgrp = lane >> 4;
+  const int K = a.k, blocks = K / 64;
+  __amdgpu_buffer_rsrc_t w[GS];
+#pragma unroll
+  for (int g = 0; g < GS; ++g) {
+    const uint16_t* wb = g / RS == 0 ? a.sw0 : a.sw1;
+    const int row = stripe * BN + wave * RS * 16 + (g % RS) * 16;
+    w[g] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(uniform_ptr(wb + (size_t)row * (size_t)K)), (short)0,
+                                             16 * K * 2, kBufferFormat);
+  }
+  const int wo[2] = {(lane >> 3) * K * 2 + (((lane & 7) ^ row_swizzle(lane >> 3)) << 4),
+                     (8 + (lane >> 3)) * K * 2 + (((lane & 7) ^ row_swizzle(8 + (lane >> 3))) << 4)};
+  uint8_t* const wring = lds + wave * GS * 2048;  // ring slot s at + s * SBLOCK
+  uint8_t* const xring = lds + SW * SBLOCK;       // stage s at + s * HSTAGE
+  auto issue_w = [&](int j, int blk, int slot) {
+    const bool in = blk < blocks;
+    load_lds_16<kNonTemporal>(w[j >> 1], wring + slot * SBLOCK + j * 1024, in ? wo[j & 1] : kOutOfRange,
+                              in ? blk * 128 : 0);
+  };
+#pragma unroll
+  for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+    for (int j = 0; j < WLOADS; ++j) issue_w(j, blk, blk);
+  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(a.sx), (short)0, (int)((int64_t)a.shared_rows * K * 2), kBufferFormat);
+  int xoff[XLOADS];
+#pragma unroll
+  for (int i = 0; i < XLOADS; ++i) {
+    const int row = 8 * (wave * XLOADS + i) + (lane >> 3);
+    const int r = r0 + (row < live ? row : 0);  // padding rows repeat a live row; their columns are dropped
+    xoff[i] = row < NCG * 16 ? r * K * 2 + (((lane & 7) ^ row_swizzle(row)) << 4) : kOutOfRange;
+  }
+  auto issue_x = [&](int j, int blk) {
+    const bool in = blk < blocks;
+    load_lds_16(xrsrc, xring + (blk & 1) * HSTAGE + (wave * XLOADS + j) * 1024, in ? xoff[j] : kOutOfRange,
+                in ? blk * 128 : 0);
+  };
+#pragma unroll
+  for (int j = 0; j < XLOADS; ++j) issue_x(j, 0);
+  f32x4 acc[TABLES][RS][NCG];
+#pragma unroll
+  for (int t = 0; t < TABLES; ++t)
+#pragma unroll
+    for (int rg = 0; rg < RS; ++rg)
+#pragma unroll
+      for (int cg = 0; cg < NCG; ++cg) acc[t][rg][cg] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int slot = 0;
+  for (int kb = 0; kb < blocks; ++kb) {
+    if (kb == 0)
+      wait_loads<0>();
+    else
+      wait_loads<WLOADS>();
+    bf16x8 A[GS][2];
+#pragma unroll
+    for (int g = 0; g < GS; ++g)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        A[g][q] = as_bf16x8(*reinterpret_cast<const u32x4*>(wring + slot * SBLOCK + g * 2048 + lrow * 128 +
+                                                            (((2 * lgrp + q) ^ row_swizzle(lrow)) << 4)));
+    barrier();
+    const int refill = slot == 0 ? SW - 1 : slot - 1;  // block kb + 2's slot
+    const uint8_t* const xl = xring + (kb & 1) * HSTAGE;
+    constexpr int P = 2 * NCG;
+    constexpr int D = P < 4 ? P : 4;    // B fragments read ahead
+    constexpr int NL = XLOADS + WLOADS;
+    bf16x8 B[P];
+    auto read_b = [&](int p) {
+      const int q = p / NCG, i = (p % NCG) * 16 + lrow;
+      B[p] = as_bf16x8(*reinterpret_cast<const u32x4*>(xl + i * kHalfRowBytes +
+                                                       (((2 * lgrp + q) ^ row_swizzle(lrow)) << 4)));
+    };
+#pragma unroll
+    for (int p = 0; p < D; ++p) read_b(p);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (p + D < P) read_b(p + D);
+      // the block's loads in order, early: one a position, or several of a small tile's
+      constexpr int PER = (NL + P - 1) / P;
+#pragma unroll
+      for (int l = p * PER; l < (p + 1) * PER && l < NL; ++l) {
+        if (l < XLOADS)
+          issue_x(l, kb + 1);
+        else
+          issue_w(l - XLOADS, kb + 2, refill);
+      }
+#pragma unroll
+      for (int g = 0; g < GS; ++g)
+        acc[g / RS][g % RS][p % NCG] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[g][p / NCG], B[p], acc[g / RS][g % RS][p % NCG], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    slot = slot + 1 == SW ? 0 : slot + 1;
+  }
+  wait_all_loads();  // the rings are idle: the epilogue reuses the LDS
+  GroupedGemmArgs o = a;
+  o.out = a.sout;
+  o.ldo = a.n;
+  o.out_rows = a.shared_rows;
+  o.outq = nullptr;
+  int orow[NCG];
+#pragma unroll
+  for (int cg = 0; cg < NCG; ++cg) orow[cg] = r0 + cg * 16 + lrow;
+  store_tile_lines<NCG, RS, TABLES, EPI, WAVES>(o, lds, acc, orow, live, wave, lane, (int64_t)stripe * BN);
+}
+
+// Rows of the shared expert's tiles: up to 256, and two tiles of up to 128 for
+// fewer rows, so that an XCD's workgroups of a 16-stripe projection are a
+// multiple of its 4 shader engines, which take them in turn.
+__host__ __device__ __forceinline__ int shared_tile_rows(int rows) {
+  return rows > 256 ? 256 : (rows + 31) / 32 * 16;
+}
+// Stripes of a projection for the shared expert's items: 256 weight rows over its tables.
+__host__ __device__ __forceinline__ int shared_stripes(int n, int tables) { return n / (256 / tables); }
+// Their workgroups, ahead of the list's (the heaviest items first): XCD x gets
+// the stripes x, x + 8, .. of every tile, an even share of them.  (Dealt in the
+// list's chunks of 32 they all fell on one or two XCDs, whose later items then
+// ended last: T=300 gate/up 924 -> 989 us; with a stripe's tiles in turn the
+// ragged last tile always fell on the same shader engine: T=777 4 % slower.)
+__host__ __device__ __forceinline__ int64_t shared_workgroups(int n, int tables, int tiles) {
+  return (int64_t)kXcds * tiles * ((shared_stripes(n, tables) + kXcds - 1) / kXcds);
+}
+
+template <int TABLES, int WAVES, int EPI>
+__device__ __forceinline__ void shared_item(const GroupedGemmArgs& a, uint8_t* lds, int b) {
+  const int stripes = shared_stripes(a.n, TABLES), per_xcd = (stripes + kXcds - 1) / kXcds;
+  const int q = b / kXcds;
+  const int stripe = b % kXcds + kXcds * (q % per_xcd), tile = q / per_xcd;
+  const int rows = shared_tile_rows(a.shared_rows);
+  const int r0 = tile * rows;
+  const int live = min(rows, a.shared_rows - r0);
+  if (stripe >= stripes || live <= 0) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int ncg = (live + 15) >> 4;
+  if (ncg == 1)
+    shared_item_run<TABLES, WAVES, EPI, 1>(a, lds, stripe, r0, live, wave, lane);
+  else if (ncg == 2)
+    shared_item_run<TABLES, WAVES, EPI, 2>(a, lds, stripe, r0, live, wave, lane);
+  else if (ncg <= 4)
+    shared_item_run<TABLES, WAVES, EPI, 4>(a, lds, stripe, r0, live, wave, lane);
+  else if (ncg <= 8)
+    shared_item_run<TABLES, WAVES, EPI, 8>(a, lds, stripe, r0, live, wave, lane);
+  else
+    shared_item_run<TABLES, WAVES, EPI, 16>(a, lds, stripe, r0, live, wave, lane);
+}
+
 template <int TABLES, int RG, int WAVES, int EPI>
 __global__ __launch_bounds__(64 * WAVES, 1) void prefill_gemm_kernel(const GroupedGemmArgs a) {
   static_assert(EPI != kEpiWeighted, "the layer's route weights are applied by the combine, not here");
@@ -437,8 +611,16 @@ __global__ __launch_bounds__(64 * WAVES, 1) void prefill_gemm_kernel(const Group
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
 
   const int stripes = a.n / BN;
+  int shared_wgs = 0;
+  if constexpr (EPI != kEpiStoreF32) {
+    shared_wgs = (int)shared_workgroups(a.n, TABLES, a.shared_tiles);
+    if ((int)blockIdx.x < shared_wgs) {
+      shared_item<TABLES, WAVES, EPI>(a, lds, blockIdx.x);
+      return;
+    }
+  }
   const int total = stripes * healthy_listings(a);
-  const int item = xcd_item(blockIdx.x, total);
+  const int item = xcd_item(blockIdx.x - shared_wgs, total);
   if (item < 0 || item >= total) return;
   // work-item scalars are workgroup-uniform: readfirstlane keeps them (and the
   // addresses derived from them) in scalar registers
@@ -1486,7 +1668,7 @@ hipError_t launch_prefill(const GroupedGemmArgs& a, hipStream_t stream) {
       allow_full_lds(reinterpret_cast<const void*>(prefill_gemm_kernel<TABLES, RG, WAVES, EPI>), lds_set);
   if (err != hipSuccess) return err;
   const int64_t items = (int64_t)(a.n / BN) * a.max_tiles;  // one stripe per item (a.stripe_run unused)
-  const int64_t grid = prefill_grid(items);
+  const int64_t grid = prefill_grid(items) + shared_workgroups(a.n, TABLES, a.shared_tiles);
   label_grouped_gemm(a, TABLES, a.tile_rows, BN, "");
   return launch_kernel(prefill_gemm_kernel<TABLES, RG, WAVES, EPI>, dim3((unsigned)grid), dim3(64 * WAVES),
                        (size_t)kPrefillLds, stream, a);
@@ -1502,6 +1684,10 @@ int prefill_stripe_run(int tables) { return tables == 2 ? kRunGateUp : kRunDown;
 
 
 int prefill_wide_tile_rows() { return kBMWide; }
+int prefill_shared_tiles(int64_t rows) {
+  const int per = shared_tile_rows((int)rows);
+  return (int)((rows + per - 1) / per);
+}
 
 // The prefill kernels hold one block scale per lane (K <= 64 blocks of 128).
 bool prefill_fits(int64_t n, int64_t k, int tables) {
@@ -1524,6 +1710,11 @@ hipError_t launch_grouped_gemm_prefill(const GroupedGemmArgs& a, int tables, int
   // a list that names wide tiles twice is for tall stripes
   if (a.wide_twice != 0 && (a.tall == 0 || a.n % prefill_tall_bn(tables) != 0)) return hipErrorInvalidValue;
   if ((a.outq != nullptr) != (a.outq_scale != nullptr)) return hipErrorInvalidValue;
+  if (a.shared_tiles != 0 &&
+      (a.xq != nullptr || epilogue == kEpiStoreF32 || a.sw0 == nullptr || (tables == 2 && a.sw1 == nullptr) ||
+       a.sx == nullptr || a.sout == nullptr || a.shared_rows <= 0 || !prefill_rows_fit(a.shared_rows, a.k) ||
+       a.shared_tiles != prefill_shared_tiles(a.shared_rows)))
+    return hipErrorInvalidValue;
   if (a.outq != nullptr && !prefill_quantizes_output(a, tables, epilogue)) return hipErrorInvalidValue;
   if (a.xq != nullptr) {
     if (a.xscale == nullptr) return hipErrorInvalidValue;

@@ -259,6 +259,15 @@ struct GroupedGemmArgs {
   int32_t tile_rows;           // routes per tile of the work list (0: unknown, up to 256)
   int32_t wide_twice;          // the work list names tiles of more than 128 routes twice (RoutePlanArgs)
   int32_t tall;                // prefill kernels: tall stripes (512 weight rows) where N allows them
+  // bf16 prefill kernel: the shared expert's work items, ahead of the list's (0 tiles: none): its
+  // bf16 tables [n, k] (sw1 with two tables), its input rows sx [shared_rows, k] and output rows
+  // sout [shared_rows, n] (the launch's epilogue), in tiles of up to 256 rows
+  const uint16_t* sw0;
+  const uint16_t* sw1;
+  const uint16_t* sx;
+  uint16_t* sout;
+  int32_t shared_rows;
+  int32_t shared_tiles;
   const char* name;            // profiler base name (null: fp8_expert_panel_matmul)
   // FP8 prefill kernel, SwiGLU epilogue on tall stripes (prefill_quantizes_output): nullable; the
   // output rows quantised for the next projection instead of stored bf16 -- e4m3 codes
@@ -299,6 +308,8 @@ hipError_t launch_grouped_gemm_wide(const GroupedGemmArgs& a, int tables, int ep
 int prefill_bn(int tables);
 int prefill_tall_bn(int tables);
 int prefill_wide_tile_rows();
+// Tiles of the shared expert's rows (GroupedGemmArgs::shared_tiles).
+int prefill_shared_tiles(int64_t rows);
 // Weight stripes one FP8 prefill work item runs for a projection of `tables` tables.
 int prefill_stripe_run(int tables);
 // Whether launch_grouped_gemm_prefill on these args runs the FP8 kernel's tall

@@ -17,8 +17,9 @@ is local and both ``psum`` of the reference are the identity.
 
 The shared expert runs inside the two decode kernels for decode shapes
 (``glm_moe_moe_layer_resident``: one pass over HBM for routed and shared
-weights), else as torch bf16 GEMMs on the same GPU (hipBLASLt), at the
-reference's rounding points; the epilogue ``routed * 2.5 + shared`` is always
+weights), inside the two prefill launches for prefill shapes of up to
+SHARED_PREFILL_ROWS_MAX rows (``glm_moe_moe_layer_shared``), else as torch bf16
+GEMMs on the same GPU (hipBLASLt), at the reference's rounding points; the epilogue ``routed * 2.5 + shared`` is always
 fused into the library's route-sum kernel.
 """
 
@@ -179,9 +180,11 @@ def routed_workspace(tokens: int, top_k: int, num_experts: int, hidden: int, int
                      device: torch.device) -> torch.Tensor:
     """The workspace of ``routed_experts`` for a call on the current stream of
     ``device``: that stream's buffer, grown when a call needs more."""
-    nbytes = max(_lib.size_query("glm_moe_routed_experts_workspace_bytes", tokens, top_k, num_experts, hidden,
-                                 intermediate), 1)
-    device = torch.device(device)
+    return _stream_workspace(max(_lib.size_query("glm_moe_routed_experts_workspace_bytes", tokens, top_k, num_experts,
+                                                 hidden, intermediate), 1), torch.device(device))
+
+
+def _stream_workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     if torch.cuda.is_current_stream_capturing() or nbytes > WORKSPACE_CACHE_MAX:
         # under HIP graph capture: a buffer of the graph's private memory pool,
         # which stays valid for every replay (a cached buffer could be regrown,
@@ -225,6 +228,7 @@ def routed_experts(
     shared: torch.Tensor | None = None,
     shared_tables: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
     routed_scale: float = 2.5,
+    _prefill_shared: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor]:
     """Routed experts of ``[T, H]`` bf16 rows: ``(bf16 [T, H], valid)``.
 
@@ -297,7 +301,8 @@ def routed_experts(
     elif out.shape != (tokens, h) or out.dtype != torch.bfloat16:
         raise ValueError("out must be bf16 [tokens, hidden]")
     valid = torch.empty((), dtype=torch.bool, device=device)
-    ws = routed_workspace(tokens, top_k, experts, h, inter, device)
+    ws = (routed_workspace(tokens, top_k, experts, h, inter, device) if _prefill_shared is None else
+          _stream_workspace(_prefill_shared_bytes(tokens, top_k, experts, h, inter), device))
     flags = 0
     if route_sum == "bfloat16":
         flags |= _lib.ROUTE_SUM_BF16
@@ -315,6 +320,10 @@ def routed_experts(
     if shared_tables is not None:
         args[15:15] = [*(_lib.ptr(t) for t in shared_tables), inter, float(routed_scale)]
         _lib.call("glm_moe_moe_layer_resident", *args, _lib.stream_of(hidden))
+    elif _prefill_shared is not None:
+        args[15:15] = [*(_lib.ptr(t) for t in _prefill_shared), float(routed_scale)]
+        args[3:3] = [None, None]
+        _lib.call("glm_moe_moe_layer_shared", *args, _lib.stream_of(hidden))
     elif shared is not None:
         args[15:15] = [_lib.ptr(shared), float(routed_scale)]
         _lib.call("glm_moe_moe_layer", *args, _lib.stream_of(hidden))
@@ -344,6 +353,7 @@ def routed_experts_from_router_logits(
     shared: torch.Tensor | None = None,
     routed_scale: float = 2.5,
     out: torch.Tensor | None = None,
+    _prefill_shared: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """Routing from the router logits, then the routed experts (and, with
     ``shared``, the fused layer epilogue): ``(bf16 [T, H], valid, route_indices,
@@ -390,9 +400,17 @@ def routed_experts_from_router_logits(
     ids = torch.empty((tokens, top_k), dtype=torch.int32, device=device)
     weights = torch.empty((tokens, top_k), dtype=torch.float32, device=device)
     valid = torch.empty((), dtype=torch.bool, device=device)
-    ws = routed_workspace(tokens, top_k, experts, h, inter, device)
     flags = ((_lib.ROUTE_SUM_BF16 if route_sum == "bfloat16" else 0) | (_lib.CHECK_WEIGHTS if check_weights else 0)
              | (_lib.FP8_ACTIVATIONS if activations == "float8_e4m3fn" else 0))
+    if _prefill_shared is not None:
+        ws = _stream_workspace(_prefill_shared_bytes(tokens, top_k, experts, h, inter), device)
+        _lib.call("glm_moe_moe_layer_shared", _lib.ptr(hidden), tokens, h, _lib.ptr(logits), _lib.ptr(bias),
+                  _lib.ptr(ids), _lib.ptr(weights), top_k, experts, inter, _lib.ptr(gate_bits), _lib.ptr(gate_scale),
+                  _lib.ptr(up_bits), _lib.ptr(up_scale), _lib.ptr(down_bits), _lib.ptr(down_scale), flags,
+                  *(_lib.ptr(t) for t in _prefill_shared), float(routed_scale), _lib.ptr(out), _lib.ptr(valid),
+                  _lib.ptr(ws), ws.numel(), _lib.stream_of(hidden))
+        return out, valid, ids, weights
+    ws = routed_workspace(tokens, top_k, experts, h, inter, device)
     _lib.call("glm_moe_moe_layer_from_router_logits", _lib.ptr(hidden), tokens, h, _lib.ptr(logits),
               _lib.ptr(bias), top_k, experts, inter, _lib.ptr(gate_bits), _lib.ptr(gate_scale), _lib.ptr(up_bits),
               _lib.ptr(up_scale), _lib.ptr(down_bits), _lib.ptr(down_scale), flags, _lib.ptr(shared),
@@ -524,6 +542,7 @@ def _shared_swiglu(hidden: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, d
 
 SHARED_ROWS_MAX = 8  # rows the few-row shared-expert kernels take (glm_moe_shared_expert_rows)
 RESIDENT_ROWS_MAX = 8  # rows whose layer runs the shared expert inside the decode kernels
+SHARED_PREFILL_ROWS_MAX = 6144  # rows whose layer runs it inside the prefill launches
 
 
 def shared_expert_rows_fit(tokens: int, hidden: int, intermediate: int) -> bool:
@@ -564,6 +583,25 @@ def _shared_expert(hidden: torch.Tensor, gate: torch.Tensor, up: torch.Tensor, d
     if shared_expert_rows_fit(hidden.shape[0], hidden.shape[1], gate.shape[0]):
         return shared_expert_rows(hidden, gate, up, down)
     return _shared_swiglu(hidden, gate, up, down)
+
+
+def _prefill_shared_bytes(tokens: int, top_k: int, experts: int, hidden: int, intermediate: int) -> int:
+    return _lib.size_query("glm_moe_moe_layer_shared_workspace_bytes", tokens, top_k, experts, hidden, intermediate)
+
+
+def _shared_in_prefill(hidden: torch.Tensor, tables, top_k: int, experts: int) -> bool:
+    """Whether the layer's prefill launches compute the shared expert too.
+
+    Up to SHARED_PREFILL_ROWS_MAX rows: GLM-5 shape, T = 9 / 61 / 128 / 777 /
+    2048 / 4000: 417 / 1042 / 1278 / 1760 / 2281 / 3385 us with the shared
+    expert's GEMMs on hipBLASLt, 387 / 1020 / 1243 / 1694 / 2252 / 3362 with its
+    rows inside; at T = 8000 its GEMMs are large enough (5667 against 5689).
+    """
+    rows, h = hidden.shape
+    return (rows <= SHARED_PREFILL_ROWS_MAX
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tables)
+            and hidden.data_ptr() % 16 == 0
+            and _prefill_shared_bytes(rows, top_k, experts, h, tables[0].shape[0]) > 0)
 
 
 def _check_layer_shapes(hidden_local, route_indices, route_weights, gate_bits, up_bits, down_bits,
@@ -665,6 +703,9 @@ def prefill_moe_from_routes(
         # two launches (its weights streamed once per group of up to 4 rows for
         # gate/up, once for down)
         shared_kw = {"shared_tables": tuple(t.contiguous() for t in tables)}
+    elif _shared_in_prefill(hidden_local, tables, contract.top_k, contract.num_experts):
+        _lib.require_device(hidden_local, *tables)
+        shared_kw = {"_prefill_shared": tables}
     else:
         shared_kw = {"shared": _shared_expert(hidden_local, *tables)}
     return routed_experts(
@@ -757,11 +798,16 @@ def prefill_moe_from_router_logits(
             check_weights=True, routed_scale=contract.routed_scaling_factor,
             shared_tables=tuple(t.contiguous() for t in tables))
     else:
+        if _shared_in_prefill(hidden_local, tables, top_k, contract.num_experts):
+            _lib.require_device(hidden_local, *tables)
+            shared_kw = {"_prefill_shared": tables}
+        else:
+            shared_kw = {"shared": _shared_expert(hidden_local, *tables)}
         out, layer_valid, ids, weights = routed_experts_from_router_logits(
             hidden_local, logits, bias, expert_gate_bits_local, expert_gate_scale_local,
             expert_up_bits_local, expert_up_scale_local, expert_down_bits_local, expert_down_scale_local,
-            top_k=top_k, route_sum="float32", check_weights=True, shared=_shared_expert(hidden_local, *tables),
-            routed_scale=contract.routed_scaling_factor)
+            top_k=top_k, route_sum="float32", check_weights=True, routed_scale=contract.routed_scaling_factor,
+            **shared_kw)
     if (torch.float64 in (router_logits.dtype, None if bias is None else correction_bias.dtype)
             or (bias is not None and bias.numel() != contract.num_experts)):
         # a finite FP64 logit may be infinite in FP32

@@ -292,6 +292,29 @@ int glm_moe_moe_layer(const uint16_t* hidden, int64_t tokens, int64_t hidden_siz
                       const uint16_t* shared, float routed_scale, uint16_t* out, uint8_t* valid,
                       void* workspace, size_t workspace_bytes, void* stream);
 
+/* glm_moe_moe_layer of prefill shapes with the shared expert computed inside the
+ * same launches from its resident bf16 tables (gate / up [intermediate,
+ * hidden_size], down [hidden_size, intermediate]), at the rounding points of
+ * glm_moe_moe_layer_resident: its rows are work items beside the experts' in the
+ * gate/up and the down launch.  With router_logits (nullable; correction_bias
+ * nullable) the layer routes first and route_indices / route_weights are
+ * outputs, as glm_moe_moe_layer_from_router_logits.  Shapes for which
+ * glm_moe_moe_layer_shared_workspace_bytes is not 0: more than the decode
+ * kernels' routes, hidden_size a multiple of 256, both sizes at most 8192,
+ * operands below 2 GiB; no FP8 mode.  Replaces prefill_moe_from_routes' shared
+ * expert and epilogue (glm_tpu/layers/moe/routed_experts.py:119-127) with the
+ * routed half (:82-117). */
+size_t glm_moe_moe_layer_shared_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t hidden,
+                                                int64_t intermediate);
+int glm_moe_moe_layer_shared(const uint16_t* hidden, int64_t tokens, int64_t hidden_size,
+                             const float* router_logits, const float* correction_bias, int32_t* route_indices,
+                             float* route_weights, int32_t top_k, int32_t num_experts, int64_t intermediate,
+                             const uint8_t* gate_bits, const float* gate_scale, const uint8_t* up_bits,
+                             const float* up_scale, const uint8_t* down_bits, const float* down_scale, uint32_t flags,
+                             const uint16_t* shared_gate, const uint16_t* shared_up, const uint16_t* shared_down,
+                             float routed_scale, uint16_t* out, uint8_t* valid, void* workspace,
+                             size_t workspace_bytes, void* stream);
+
 /* 1 when a layer of this geometry runs on the decode kernels (tokens * top_k
  * <= 64 and the hidden / intermediate sizes they stage), the shapes
  * glm_moe_moe_layer_resident takes; else 0.  Host-only query, no reference

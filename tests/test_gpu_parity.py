@@ -552,6 +552,59 @@ def test_resident_shared_expert_layer(device, tokens, experts, hidden, inter, to
     np.testing.assert_array_equal(bf16_bits_of(again), bf16_bits_of(got))  # deterministic
 
 
+# The shared expert inside the prefill launches: one tile of one group, tiles of
+# every variant (1, 2, 4, 8, 16 groups, full and ragged), several tiles, stripe
+# counts that leave XCDs without one (3 gate/up and 5 down stripes, 2 and 1), one
+# K block of 64 pairs per projection size, tall stripes beside them.
+@pytest.mark.parametrize("tokens,experts,hidden,inter,top_k", [
+    (9, 16, 512, 256, 8), (33, 16, 1280, 384, 4), (61, 16, 256, 256, 4), (128, 16, 512, 128, 4),
+    (129, 8, 1280, 384, 2), (256, 8, 512, 256, 2), (257, 8, 512, 256, 2), (530, 8, 768, 384, 2),
+    (1000, 64, 512, 1792, 8),
+])
+def test_shared_expert_in_the_prefill_launches(device, tokens, experts, hidden, inter, top_k):
+    from glm_moe.contracts import single_gpu_contract
+    from glm_moe.layers.moe.routed_experts import (_shared_in_prefill, prefill_moe_from_router_logits,
+                                                   prefill_moe_from_routes)
+    from glm_moe.layers.moe.router import route_glm_noaux_tc_logits
+
+    cfg, x, ids, w, tables = _small_case(tokens, experts, hidden, inter, top_k, 0.0, seed=tokens + 190)
+    t = _device_tables(tables, device)
+    rng = np.random.default_rng(tokens)
+    shared_f32 = [O.bf16_round((rng.standard_normal(shape) * std).astype(np.float32))
+                  for shape, std in (((inter, hidden), hidden ** -0.5), ((inter, hidden), hidden ** -0.5),
+                                     ((hidden, inter), 2 * inter ** -0.5))]
+    shared_dev = [bf16_dev(a, device) for a in shared_f32]
+    contract = single_gpu_contract(hidden_size=hidden, intermediate_size=inter, num_experts=experts, top_k=top_k)
+    x_dev = bf16_dev(x, device)
+    tabs = [t[k] for k in TABLE_KEYS]
+    assert _shared_in_prefill(x_dev, shared_dev, top_k, experts)
+    got, ok = prefill_moe_from_routes(x_dev, dev(ids, device), dev(w, device), *tabs, *shared_dev, contract=contract)
+    ref, ref_ok, mag = O.moe_layer(x, ids, w, **tables, shared_gate=shared_f32[0], shared_up=shared_f32[1],
+                                   shared_down=shared_f32[2], return_magnitude=True)
+    assert bool(ok) == ref_ok
+    print(cfg, assert_moe_close(host_f32(got), ref, magnitude=mag, flip_ulps=closeness.LAYER_FLIP_ULPS,
+                                max_flips=closeness.layer_max_flips(ref.size)))
+    # tables the launches do not take (views with other strides) run on the GEMMs: equal up to FP32 order
+    views = [a.t().contiguous().t() for a in shared_dev]
+    assert not _shared_in_prefill(x_dev, views, top_k, experts)
+    other, _ = prefill_moe_from_routes(x_dev, dev(ids, device), dev(w, device), *tabs, *views, contract=contract)
+    assert_moe_close(host_f32(got), host_f32(other), magnitude=mag, label="vs hipBLASLt",
+                     flip_ulps=closeness.LAYER_FLIP_ULPS, max_flips=closeness.layer_max_flips(ref.size))
+    # from router logits: the same layer bit for bit
+    logits = torch.randn((tokens, experts), generator=torch.Generator().manual_seed(tokens)).to(device)
+    bias = torch.zeros(experts, device=device)
+    out, l_ids, l_w, row_ok = prefill_moe_from_router_logits(x_dev, logits, bias, *tabs, *shared_dev,
+                                                             contract=contract)
+    r_ids, r_w = route_glm_noaux_tc_logits(logits, bias, top_k=top_k)
+    want, _ = prefill_moe_from_routes(x_dev, r_ids, r_w, *tabs, *shared_dev, contract=contract)
+    assert torch.equal(l_ids, r_ids) and torch.equal(l_w, r_w) and torch.equal(out, want) and bool(row_ok.all())
+    # a non-finite shared row clears health
+    broken = [a.clone() for a in shared_dev]
+    broken[2][0, 0] = float("inf")
+    _, ok = prefill_moe_from_routes(x_dev, dev(ids, device), dev(w, device), *tabs, *broken, contract=contract)
+    assert not bool(ok)
+
+
 def test_resident_shared_expert_nonfinite_clears_health(device):
     from glm_moe.layers.moe.routed_experts import routed_experts
 
