@@ -126,6 +126,36 @@ __global__ void zero_rows_kernel(uint32_t* out, int64_t rows, int64_t row_words,
   }
 }
 
+// Eight columns of one route row into a token's sum, with the bf16 route weight
+// (routed_experts.py:104-105): bf16(bf16(down) * bf16(w)).
+__device__ __forceinline__ void add_route(float (&acc)[8], const u32x4& v, float w, bool weighted) {
+  w = round_to_bf16(w);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float lo = bf16_bits_to_f32(v[j] & 0xFFFFu), hi = bf16_bits_to_f32(v[j] >> 16);
+    if (weighted) {
+      lo = round_to_bf16(lo * w);
+      hi = round_to_bf16(hi * w);
+    }
+    acc[2 * j] += lo;
+    acc[2 * j + 1] += hi;
+  }
+}
+// The layer epilogue on eight columns: false where one is not finite.
+__device__ __forceinline__ bool add_shared(float (&acc)[8], const uint16_t* shared, float routed_scale) {
+  const u32x4 sv = *reinterpret_cast<const u32x4*>(shared);
+  bool finite = true;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    acc[2 * j] = round_to_bf16(round_to_bf16(round_to_bf16(acc[2 * j]) * routed_scale) +
+                               bf16_bits_to_f32(sv[j] & 0xFFFFu));
+    acc[2 * j + 1] = round_to_bf16(round_to_bf16(round_to_bf16(acc[2 * j + 1]) * routed_scale) +
+                                   bf16_bits_to_f32(sv[j] >> 16));
+    finite &= isfinite(acc[2 * j]) && isfinite(acc[2 * j + 1]);
+  }
+  return finite;
+}
+
 // FP32 sum of a token's top-k weighted route rows in slot order, one bf16
 // rounding (routed_experts.py:106-117; also the decode body's per-owner bf16
 // sum, :293, which JAX computes in FP32 and rounds once).  With ids given, a slot whose raw expert id lies outside [0, experts) is not
@@ -170,33 +200,10 @@ __global__ void combine_routes_kernel(const uint16_t* y, int64_t tokens, int32_t
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         if (u >= n) break;
-        // bf16 route weight (routed_experts.py:104-105): bf16(bf16(down) * bf16(w))
-        w[u] = round_to_bf16(w[u]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float lo = bf16_bits_to_f32(v[u][j] & 0xFFFFu), hi = bf16_bits_to_f32(v[u][j] >> 16);
-          if (route_w != nullptr) {
-            lo = round_to_bf16(lo * w[u]);
-            hi = round_to_bf16(hi * w[u]);
-          }
-          acc[2 * j] += lo;
-          acc[2 * j + 1] += hi;
-        }
+        add_route(acc, v[u], w[u], route_w != nullptr);
       }
     }
-    if (shared != nullptr) {
-      const u32x4 sv = *reinterpret_cast<const u32x4*>(shared + t * h + c);
-      bool finite = true;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        acc[2 * j] = round_to_bf16(round_to_bf16(round_to_bf16(acc[2 * j]) * routed_scale) +
-                                   bf16_bits_to_f32(sv[j] & 0xFFFFu));
-        acc[2 * j + 1] = round_to_bf16(round_to_bf16(round_to_bf16(acc[2 * j + 1]) * routed_scale) +
-                                       bf16_bits_to_f32(sv[j] >> 16));
-        finite &= isfinite(acc[2 * j]) && isfinite(acc[2 * j + 1]);
-      }
-      if (!finite) valid[0] = 0;
-    }
+    if (shared != nullptr && !add_shared(acc, shared + t * h + c, routed_scale)) valid[0] = 0;
     if (out_f32 != nullptr) {
       // a share's partial for the caller's sum over the expert axis
       f32x4 lo4, hi4;
@@ -209,6 +216,48 @@ __global__ void combine_routes_kernel(const uint16_t* y, int64_t tokens, int32_t
       *reinterpret_cast<f32x4*>(out_f32 + t * h + c + 4) = hi4;
       continue;
     }
+    u32x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
+    *reinterpret_cast<u32x4*>(out + t * h + c) = o;
+  }
+}
+
+// The same where every route is owned and the output is bf16 (a whole layer):
+// a workgroup takes one token's columns (part blockIdx.x of a token's), so the
+// weights are scalars, no id is read, and no thread divides; the route rows,
+// each read once, are loaded past the caches' reuse.  Bound by HBM: 777 tokens
+// of 8 x 12 KB 22.6 -> 18.9 us (5 TB/s), the T=2048 GLM-5-shape layer 2216 ->
+// 2205.  Not for shares: with about one owned row a token, whose id is read
+// first, the workgroups are a chain of latencies (2048 tokens, one of eight
+// shares: 41 us against the kernel above's 23.5).
+__global__ __launch_bounds__(256) void combine_all_routes_kernel(const uint16_t* y, int64_t tokens, int32_t top_k,
+                                                                 int64_t h, const float* route_w,
+                                                                 const uint16_t* shared, float routed_scale,
+                                                                 uint8_t* valid, uint16_t* out) {
+  const int64_t c = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;
+  if (c >= h) return;
+  for (int64_t t = blockIdx.y; t < tokens; t += gridDim.y) {
+    const uint16_t* const rows = y + t * top_k * h + c;
+    float acc[8] = {};
+    for (int s0 = 0; s0 < top_k; s0 += 8) {
+      const int n = min(top_k - s0, 8);
+      u32x4 v[8];
+      float w[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if (u < n) {
+          v[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(rows + (s0 + u) * h));
+          w[u] = route_w != nullptr ? route_w[t * top_k + s0 + u] : 1.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        if (u >= n) break;
+        add_route(acc, v[u], w[u], route_w != nullptr);
+      }
+    }
+    if (shared != nullptr && !add_shared(acc, shared + t * h + c, routed_scale)) valid[0] = 0;
     u32x4 o;
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = pack_bf16x2(acc[2 * j], acc[2 * j + 1]);
@@ -551,6 +600,15 @@ hipError_t launch_combine_routes(const uint16_t* y, int64_t tokens, int32_t top_
     return hipErrorInvalidValue;
   label_next_launch("restore_prefill_route_rows_t%lld_k%d_h%lld%s", (long long)tokens, top_k, (long long)h,
                     shared != nullptr ? "_epilogue" : "");
+  if (ids == nullptr && out_f32 == nullptr) {
+    // a token's columns in equal parts of up to 256 threads
+    const int64_t groups = h / 8, parts = (groups + 255) / 256;
+    const int64_t threads = ((groups + parts - 1) / parts + 63) / 64 * 64;
+    if (parts > INT32_MAX / 256) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)((groups + threads - 1) / threads), (unsigned)(tokens < 65535 ? tokens : 65535));
+    return launch_kernel(combine_all_routes_kernel, grid, dim3((unsigned)threads), 0, stream, y, tokens, top_k, h,
+                         route_w, shared, routed_scale, valid, out);
+  }
   return launch_kernel(combine_routes_kernel, grid_for(total, 256), dim3(256), 0, stream, y, tokens,
                      top_k, h, ids, own, route_w, shared, routed_scale, valid, out, out_f32, round_partial);
 }

@@ -1192,6 +1192,36 @@ def test_expert_share_at_production_size_matches_owned_partial(device, productio
     print(f"share {rank}: {int(owned_rows.sum())} rows", assert_moe_close(got, ref))
 
 
+@pytest.mark.parametrize("tokens,experts,hidden,inter,top_k,shares", [
+    (70, 16, 512, 256, 16, 1),   # two groups of eight slots
+    (40, 24, 768, 256, 11, 3),   # a second group of three slots, some of them unowned in a share
+    (30, 12, 2560, 256, 5, 4),   # two workgroups a token, the second with empty lanes
+    (33, 8, 256, 128, 3, 2),     # a token's columns in less than a wave
+])
+def test_route_combine_splits(device, tokens, experts, hidden, inter, top_k, shares):
+    """The combine's column parts, slot groups and owned masks: whole layers
+    and FP32 shares against the oracle."""
+    from glm_moe.layers.moe.routed_experts import routed_experts, routed_experts_share
+
+    cfg, x, ids, w, tables = _small_case(tokens, experts, hidden, inter, top_k, 0.0, seed=tokens + 61)
+    t = _device_tables(tables, device)
+    xs, idd, wd = bf16_dev(x, device), dev(ids, device), dev(w, device)
+    for route_sum in ("float32", "bfloat16"):
+        out, ok = routed_experts(xs, idd, wd, *(t[k] for k in TABLE_KEYS), route_sum=route_sum)
+        assert bool(ok)
+        ref, _ = O.routed_experts(x, ids, w, **tables, route_sum=route_sum)
+        print(cfg, route_sum, assert_moe_close(host_f32(out), ref))
+    own = experts // shares
+    for rank in range(shares):
+        lo = own * rank
+        part, ok = routed_experts_share(xs, idd, wd, *(t[k][lo:lo + own] for k in TABLE_KEYS), num_experts=experts,
+                                        expert_offset=lo)
+        assert bool(ok)
+        ref, _ = O.routed_experts(x, ids, w, **{k: v[lo:lo + own] for k, v in tables.items()}, num_experts=experts,
+                                  expert_offset=lo, round_output=False)
+        print(f"share {rank}", assert_moe_close(host_f32(part), ref))
+
+
 @pytest.mark.parametrize("tokens,top_k", [(300, 6), (4, 8), (1, 8)])
 def test_expert_shares_sum_to_the_whole_layer(device, tokens, top_k):
     """Four shares of 16 experts: each partial matches the oracle's share, the
