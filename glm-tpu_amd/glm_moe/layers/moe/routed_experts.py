@@ -751,6 +751,9 @@ def prefill_moe_from_router_logits(
                          "with route_glm_noaux_tc_logits and call prefill_moe_from_routes")
     if router_logits.ndim != 2 or router_logits.shape != (hidden_local.shape[0], contract.num_experts):
         raise ValueError(f"router_logits must have shape {(hidden_local.shape[0], contract.num_experts)}")
+    if correction_bias is not None and correction_bias.numel() != contract.num_experts:
+        # the router kernels read one value per expert
+        raise ValueError(f"correction_bias must have shape {(contract.num_experts,)}")
     top_k = contract.top_k
     inter, h = contract.intermediate_size, contract.hidden_size
     _check_layer_shapes(hidden_local, None, None, expert_gate_bits_local, expert_up_bits_local,
@@ -785,8 +788,7 @@ def prefill_moe_from_router_logits(
             *(_lib.ptr(t) for t in resident), inter, float(contract.routed_scaling_factor), _lib.ptr(ids),
             _lib.ptr(weights), _lib.ptr(out), _lib.ptr(layer_valid), _lib.ptr(ws), ws.numel(),
             _lib.stream_of(hidden_local))
-    elif decode and rows > 1 and correction_bias is not None and correction_bias.shape == (
-            contract.num_experts,):
+    elif decode and rows > 1 and correction_bias is not None:
         # a few rows: the router kernel, then the decode kernels with the resident
         # shared expert (its weights streamed once per group of up to 4 rows)
         from glm_moe.layers.moe.router import route_glm_noaux_tc_logits
@@ -808,8 +810,7 @@ def prefill_moe_from_router_logits(
             expert_up_bits_local, expert_up_scale_local, expert_down_bits_local, expert_down_scale_local,
             top_k=top_k, route_sum="float32", check_weights=True, routed_scale=contract.routed_scaling_factor,
             **shared_kw)
-    if (torch.float64 in (router_logits.dtype, None if bias is None else correction_bias.dtype)
-            or (bias is not None and bias.numel() != contract.num_experts)):
+    if torch.float64 in (router_logits.dtype, None if bias is None else correction_bias.dtype):
         # a finite FP64 logit may be infinite in FP32
         row_valid = torch.isfinite(router_logits).all(dim=1) & torch.isfinite(weights).all(dim=1) & layer_valid
         return out, ids, weights, row_valid if bias is None else row_valid & torch.isfinite(correction_bias).all()

@@ -278,3 +278,35 @@ def test_bench_reads_measured_traffic_from_the_profiles():
         base, _, mode = name.partition(":")
         assert base in S.CONFIGS and mode in ("", "fp8"), name
         assert rec["bytes"] > 0 and rec["source"].startswith("profiles/")
+
+
+def _layer_on_cpu(rows, **other):
+    """Arguments of prefill_moe_from_router_logits on the CPU (a call that passes the host's checks is
+    refused for its device): 8 experts of 256 x 256, top-2."""
+    from glm_moe.contracts import single_gpu_contract
+
+    e, h, i = 8, 256, 256
+    args = dict(
+        hidden_local=torch.zeros(rows, h, dtype=torch.bfloat16), router_logits=torch.zeros(rows, e),
+        correction_bias=torch.zeros(e), expert_gate_bits_local=torch.zeros(e, i, h, dtype=torch.uint8),
+        expert_gate_scale_local=torch.ones(e, i // 128, h // 128),
+        expert_up_bits_local=torch.zeros(e, i, h, dtype=torch.uint8),
+        expert_up_scale_local=torch.ones(e, i // 128, h // 128),
+        expert_down_bits_local=torch.zeros(e, h, i, dtype=torch.uint8),
+        expert_down_scale_local=torch.ones(e, h // 128, i // 128),
+        shared_gate_local=torch.zeros(i, h, dtype=torch.bfloat16), shared_up_local=torch.zeros(i, h, dtype=torch.bfloat16),
+        shared_down_local=torch.zeros(h, i, dtype=torch.bfloat16))
+    contract = single_gpu_contract(hidden_size=h, intermediate_size=i, num_experts=e, top_k=2)
+    return {**args, **other, "contract": contract}
+
+
+@pytest.mark.parametrize("rows", [1, 3, 9])
+@pytest.mark.parametrize("length", [1, 7, 9])
+def test_layer_from_router_logits_refuses_a_bias_of_another_length(rows, length):
+    # the router kernels read the bias of every expert: a shorter one is not read at all
+    from glm_moe.layers.moe.routed_experts import prefill_moe_from_router_logits
+
+    with pytest.raises(ValueError, match="correction_bias must have shape"):
+        prefill_moe_from_router_logits(**_layer_on_cpu(rows, correction_bias=torch.zeros(length)))
+    with pytest.raises(ValueError, match="GPU tensors only"):
+        prefill_moe_from_router_logits(**_layer_on_cpu(rows))
