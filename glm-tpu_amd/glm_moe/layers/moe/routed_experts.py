@@ -771,6 +771,12 @@ def prefill_moe_from_router_logits(
     if decode and rows == 1 and contract.num_experts <= 256:
         # one row: the resident shared expert inside the two decode kernels, which also route
         experts = contract.num_experts
+        if any(t.dtype != torch.bfloat16 for t in tables):
+            raise ValueError("resident shared expert tables must be contiguous bf16 [I, H], [I, H], [H, I]")
+        for scale, n, k in ((expert_gate_scale_local, inter, h), (expert_up_scale_local, inter, h),
+                            (expert_down_scale_local, h, inter)):
+            if scale.dtype != torch.float32 or scale.shape != (experts, n // 128, k // 128):
+                raise ValueError("expert scales must be float32 [E, N/128, K/128]")
         resident = tuple(t.contiguous() for t in tables)
         _lib.require_device(hidden_local, logits, bias, expert_gate_bits_local, expert_gate_scale_local,
                             expert_up_bits_local, expert_up_scale_local, expert_down_bits_local,

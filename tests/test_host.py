@@ -310,3 +310,28 @@ def test_layer_from_router_logits_refuses_a_bias_of_another_length(rows, length)
         prefill_moe_from_router_logits(**_layer_on_cpu(rows, correction_bias=torch.zeros(length)))
     with pytest.raises(ValueError, match="GPU tensors only"):
         prefill_moe_from_router_logits(**_layer_on_cpu(rows))
+
+
+@pytest.mark.parametrize("rows", [1, 3])
+@pytest.mark.parametrize("operand,wrong,match", [
+    ("expert_gate_scale_local", torch.ones(8, 2, 1), "expert scales must be float32"),
+    ("expert_up_scale_local", torch.ones(1), "expert scales must be float32"),
+    ("expert_down_scale_local", torch.ones(8, 2, 2, dtype=torch.bfloat16), "expert scales must be float32"),
+    ("shared_gate_local", torch.zeros(256, 256, dtype=torch.uint8), "tables must be contiguous bf16"),
+    ("shared_down_local", torch.zeros(256, 256, dtype=torch.float32), "tables must be contiguous bf16"),
+])
+def test_layer_from_router_logits_checks_every_operand_the_kernels_read(rows, operand, wrong, match):
+    # the one-row call reaches the library directly, the few-row one through routed_experts
+    from glm_moe.layers.moe.routed_experts import prefill_moe_from_router_logits, routed_experts
+
+    args = _layer_on_cpu(rows, **{operand: wrong})
+    if rows == 1:
+        with pytest.raises(ValueError, match=match):
+            prefill_moe_from_router_logits(**args)
+        return
+    tables = [args[n] for n in ("expert_gate_bits_local", "expert_gate_scale_local", "expert_up_bits_local",
+                                "expert_up_scale_local", "expert_down_bits_local", "expert_down_scale_local")]
+    with pytest.raises(ValueError, match=match):
+        routed_experts(args["hidden_local"], torch.zeros(rows, 2, dtype=torch.int32), torch.ones(rows, 2), *tables,
+                       shared_tables=tuple(args[n] for n in ("shared_gate_local", "shared_up_local",
+                                                             "shared_down_local")))
