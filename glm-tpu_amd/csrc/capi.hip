@@ -925,7 +925,12 @@ int glm_moe_routed_projection(const uint16_t* lhs, int32_t slots, int64_t k, int
     return fail(GLM_MOE_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given",
                 glm_moe_routed_projection_workspace_bytes(slots), workspace_bytes);
   hipStream_t s = as_stream(stream);
-  if (routed_projection_fits(n, k)) {
+  // the decode streams read buffers, and the rows of two slots of one expert go
+  // straight into LDS, 16 bytes a lane: rows or tables that are not 16-byte
+  // aligned keep the tiles, whose plain loads take any address
+  const bool aligned = ((reinterpret_cast<uintptr_t>(lhs) | reinterpret_cast<uintptr_t>(bits0) |
+                         (tables == 2 ? reinterpret_cast<uintptr_t>(bits1) : 0)) & 15) == 0;
+  if (aligned && routed_projection_fits(n, k)) {
     const uint8_t* const bits[2] = {bits0, bits1};
     const float* const scale[2] = {scale0, scale1};
     GLM_HIP(launch_routed_projection(lhs, slots, (int32_t)k, tables, bits, scale, experts, (int32_t)n,

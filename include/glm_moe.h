@@ -164,7 +164,8 @@ int glm_moe_panel_fp8_matmul_ws(const uint16_t* lhs, int64_t m, int64_t k, const
 /* Replaces glm_tpu/kernels/fp8_grouped_matmul/kernel.py:125-299 fp8_routed_projection:
  * one bf16 row per route slot lhs [slots, k] against the slot's expert
  * (ids clipped to [0, experts)) in 1 or 2 tables; out [slots, tables, n] f32 or bf16;
- * unowned slots are zero.  Needs glm_moe_routed_projection_workspace_bytes(slots). */
+ * unowned slots are zero.  Needs glm_moe_routed_projection_workspace_bytes(slots),
+ * which calls with k above 8192 or lhs or bits not 16-byte aligned use. */
 size_t glm_moe_routed_projection_workspace_bytes(int32_t slots);
 int glm_moe_routed_projection(const uint16_t* lhs, int32_t slots, int64_t k, int32_t tables,
                               const uint8_t* bits0, const float* scale0, const uint8_t* bits1,

@@ -415,6 +415,38 @@ def test_routed_projection_slots_match_oracle(device, slots, experts, n, k, tabl
     np.testing.assert_allclose(actual, ref, rtol=1e-5, atol=8 * 2**-24 * np.sqrt(k) * np.abs(ref).max())
 
 
+# Contiguous views whose first element is not 16-byte aligned, slots that share an
+# expert and slots alone: rows, tables and both off by one element.
+@pytest.mark.parametrize("row_offset,table_offset", [(1, 0), (0, 1), (3, 5)])
+@pytest.mark.parametrize("tables", [1, 2])
+def test_routed_projection_takes_unaligned_views(device, tables, row_offset, table_offset):
+    from glm_moe.kernels.fp8_grouped_matmul.kernel import RoutedProjectionConfig, fp8_routed_projection
+
+    def at(offset, t):
+        flat = torch.zeros(t.numel() + 16, dtype=t.dtype, device=device)
+        view = flat[offset:offset + t.numel()].view(t.shape)
+        view.copy_(t)
+        return view
+
+    rng = np.random.default_rng(row_offset + 10 * table_offset)
+    slots, experts, n, k = 7, 3, 256, 640
+    x = O.bf16_round(rng.normal(0, 0.2, (slots, k)).astype(np.float32))
+    pairs = []
+    for _ in range(tables):
+        bits = torch.from_numpy(rng.normal(0, 0.15, (experts, n, k)).astype(np.float32)).to(
+            torch.float8_e4m3fn).view(torch.uint8).numpy()
+        pairs.append((bits, rng.uniform(0.1, 2.0, (experts, n // 128, k // 128)).astype(np.float32)))
+    ids = np.array([0, 1, 0, 2, 1, 1, 0], np.int32)
+    owned = np.array([1, 1, 1, 1, 0, 1, 1], bool)
+    got = fp8_routed_projection(
+        at(row_offset, bf16_dev(x, device)),
+        tuple((at(table_offset, dev(b, device)), dev(s, device)) for b, s in pairs), dev(ids, device),
+        dev(owned, device), config=RoutedProjectionConfig(output_tile=256, contraction_tile=128))
+    ref = O.routed_projection(x, tuple(pairs), ids, owned, result_dtype="float32")
+    # FP32 sums of K exact products in another order (as the panel tiles' bound)
+    np.testing.assert_allclose(host_f32(got), ref, rtol=1e-5, atol=8 * 2**-24 * np.sqrt(k) * np.abs(ref).max())
+
+
 # ----------------------------------------------------------------------------- routed experts
 @pytest.fixture(scope="module")
 def golden():
