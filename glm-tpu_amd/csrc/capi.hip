@@ -1090,6 +1090,10 @@ int glm_moe_moe_layer_shared(const uint16_t* hidden, int64_t tokens, int64_t hid
                              float routed_scale, uint16_t* out, uint8_t* valid, void* workspace,
                              size_t workspace_bytes, void* stream) {
   GLM_REQUIRE(shared_gate && shared_up && shared_down, "null shared expert table");
+  // the shared expert's items load both straight into LDS, 16 bytes a lane
+  GLM_REQUIRE(((reinterpret_cast<uintptr_t>(hidden) | reinterpret_cast<uintptr_t>(shared_gate) |
+                reinterpret_cast<uintptr_t>(shared_up) | reinterpret_cast<uintptr_t>(shared_down)) & 15) == 0,
+              "hidden rows and shared expert tables must be 16-byte aligned");
   GLM_REQUIRE(std::isfinite(routed_scale), "routed scale must be finite");
   GLM_REQUIRE(router_logits == nullptr || top_k <= kWave,
               "the GPU router selects at most %d experts per token (one wave lane each)", kWave);

@@ -302,7 +302,8 @@ int glm_moe_moe_layer(const uint16_t* hidden, int64_t tokens, int64_t hidden_siz
  * outputs, as glm_moe_moe_layer_from_router_logits.  Shapes for which
  * glm_moe_moe_layer_shared_workspace_bytes is not 0: more than the decode
  * kernels' routes, hidden_size a multiple of 256, both sizes at most 8192,
- * operands below 2 GiB; no FP8 mode.  Replaces prefill_moe_from_routes' shared
+ * operands below 2 GiB; no FP8 mode.  hidden and the shared tables are 16-byte
+ * aligned (else GLM_MOE_ERR_ARGUMENT).  Replaces prefill_moe_from_routes' shared
  * expert and epilogue (glm_tpu/layers/moe/routed_experts.py:119-127) with the
  * routed half (:82-117). */
 size_t glm_moe_moe_layer_shared_workspace_bytes(int64_t tokens, int32_t top_k, int32_t num_experts, int64_t hidden,

@@ -335,3 +335,22 @@ def test_layer_from_router_logits_checks_every_operand_the_kernels_read(rows, op
         routed_experts(args["hidden_local"], torch.zeros(rows, 2, dtype=torch.int32), torch.ones(rows, 2), *tables,
                        shared_tables=tuple(args[n] for n in ("shared_gate_local", "shared_up_local",
                                                              "shared_down_local")))
+
+
+@pytest.mark.parametrize("operand", [None, 0, 1, 2, 3])
+def test_shared_expert_in_the_launches_refuses_unaligned_operands(operand):
+    # hidden and the shared tables go straight into LDS, 16 bytes a lane: refused before any launch
+    from glm_moe import _lib
+
+    lib = _lib.lib()
+    null, fake = ctypes.c_void_p(0), ctypes.c_void_p(4096)
+    at = [ctypes.c_void_p(4096 + (2 if i == operand else 0)) for i in range(4)]
+    status = lib.glm_moe_moe_layer_shared(
+        at[0], 300, 6144, null, null, fake, fake, 8, 256, 2048, fake, fake, fake, fake, fake, fake, 0, at[1], at[2],
+        at[3], ctypes.c_float(2.5), fake, fake, fake, 0, null)
+    if operand is None:  # the next check: the workspace
+        assert status == _lib.ERR_WORKSPACE
+        return
+    assert status == _lib.ERR_ARGUMENT
+    with pytest.raises(ValueError, match="16-byte aligned"):
+        _lib.check(status)
