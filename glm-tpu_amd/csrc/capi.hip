@@ -126,17 +126,26 @@ int compute_units() {
 //     shape, T=9 / 64 / 256: +7 / +3.5 / +1 %; from 16 to 48 routes an expert
 //     the two are within 2 %, evenly popular experts slightly for 256-row
 //     stripes, skewed ones for tall; T=2048: tall 2266, 256-row 2291 us);
-//   * the gate/up items fill 2.5 rounds of the CUs, so that the last round
-//     costs little (32 of 256 experts, one or two rounds: T=2048 / 4000 tall
-//     361 / 528 us, 256-row 314 / 500; 64 of 256, two to three rounds: 583 /
-//     833, 543 / 864).  An expert has at least one listing, a skewed routing
-//     about 1.5 listings per 128 routes.
+//   * the gate/up items fill more than two rounds of the CUs, so that the last
+//     round costs little.  An expert has at least one listing, a skewed routing
+//     about 1.5 listings per 128 routes.  Measured in means over even routings
+//     and ones skewed by a bias of N(0, 0.05), tall / 256-row us: up to two
+//     rounds, 32 of 256 experts T=1024 263 / 254, T=2048 356 / 332, T=3000 420 /
+//     406, 64 of 256 T=1500 567 / 524, T=2048 606 / 588 (evenly popular 508 /
+//     522), 32 of 128 experts, H 4096, I 1536, T=2500 315 / 291; from two to 2.5,
+//     that one at T=3700 374 / 381, T=4000 385 / 402 (evenly popular 389 / 468:
+//     each expert one full tile, some a second of a few routes), 64 of 256 T=3000
+//     714 / 718 (595 / 626), 32 of 256 T=6000 604 / 599, but 128 experts, H 2048,
+//     I 768, T=2000 268 / 248: 534 tall items, a third round of 22.  A single
+//     routing moves either by 10 % as its tiles happen to fill rounds: 24 of the
+//     T=2048 share, 256-row 290 .. 385, tall 300 .. 408.  Graph replay and loops
+//     of calls agree within 1 % on each.
 bool bf16_tall_stripes(int64_t routes, int64_t global_experts, int64_t experts, int64_t hidden,
                        int64_t intermediate) {
   if (routes < 16 * global_experts || intermediate % prefill_tall_bn(2) != 0 || hidden % prefill_tall_bn(1) != 0)
     return false;
   const int64_t listings = std::max(experts, routes * experts / global_experts * 3 / 256);
-  return 2 * listings * (intermediate / prefill_tall_bn(2)) >= 5 * (int64_t)compute_units();
+  return listings * (intermediate / prefill_tall_bn(2)) > 2 * (int64_t)compute_units();
 }
 
 // Panels of the reference's kernel: 32 rows.
@@ -150,7 +159,8 @@ bool panel_matmul_on_tiles(int64_t m, int64_t k, int32_t groups, int64_t n) {
   return m > 0 && k > 0 && groups > 0 && n > 0 && prefill_fits(n, k, 1) && prefill_rows_fit(m, k) &&
          m * k >= ((int64_t)1 << 29) / n;
 }
-// Its stripes, by bf16_tall_stripes' rule for one table.
+// Its stripes: tall from 16 rows a group and 2.5 rounds of its items on (one
+// table, a call of its own: not measured against bf16_tall_stripes' two).
 bool panel_tall_stripes(int64_t rows, int64_t groups, int64_t n) {
   return rows >= 16 * groups && n % prefill_tall_bn(1) == 0 &&
          2 * std::max(groups, rows * 3 / 256) * (n / prefill_tall_bn(1)) >= 5 * (int64_t)compute_units();
@@ -1111,6 +1121,17 @@ int glm_moe_uses_decode_kernels(int64_t tokens, int32_t top_k, int64_t hidden_si
                  uses_decode_path(tokens * top_k, hidden_size, intermediate)
              ? 1
              : 0;
+}
+
+int glm_moe_prefill_stripe_rows(int64_t tokens, int32_t top_k, int32_t local_experts, int32_t num_experts,
+                                int64_t hidden_size, int64_t intermediate) {
+  if (tokens <= 0 || top_k <= 0 || local_experts <= 0 || num_experts < local_experts || hidden_size <= 0 ||
+      intermediate <= 0 || tokens > INT32_MAX / 2 / top_k ||
+      !on_prefill_kernel(tokens, top_k, local_experts, hidden_size, intermediate))
+    return 0;
+  return bf16_tall_stripes(tokens * top_k, num_experts, local_experts, hidden_size, intermediate)
+             ? prefill_tall_bn(1)
+             : prefill_bn(1);
 }
 
 int glm_moe_moe_layer_resident(const uint16_t* hidden, int64_t tokens, int64_t hidden_size,

@@ -96,6 +96,7 @@ SIGNATURES: dict[str, tuple] = {
          _vp, _vp, _vp, _sz, _vp],
     ),
     "glm_moe_uses_decode_kernels": (ctypes.c_int, [_i64, _i32, _i64, _i64]),
+    "glm_moe_prefill_stripe_rows": (ctypes.c_int, [_i64, _i32, _i32, _i32, _i64, _i64]),
     "glm_moe_moe_layer_resident": (
         ctypes.c_int,
         [_vp, _i64, _i64, _vp, _vp, _i32, _i32, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _u32, _vp, _vp, _vp, _i64, _f,

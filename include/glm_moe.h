@@ -323,6 +323,13 @@ int glm_moe_moe_layer_shared(const uint16_t* hidden, int64_t tokens, int64_t hid
  * counterpart (the reference picks its layer body by program, not by shape). */
 int glm_moe_uses_decode_kernels(int64_t tokens, int32_t top_k, int64_t hidden_size, int64_t intermediate);
 
+/* Weight rows of a work item of a bf16 layer's prefill projections, 512 (tall
+ * stripes) or 256, for a call with the tables of local_experts of num_experts
+ * on the current device; 0 where the layer does not run on the prefill
+ * kernels.  Host-only query, no reference counterpart. */
+int glm_moe_prefill_stripe_rows(int64_t tokens, int32_t top_k, int32_t local_experts, int32_t num_experts,
+                                int64_t hidden_size, int64_t intermediate);
+
 /* The whole decode MoE layer in two kernels: glm_moe_moe_layer with the
  * shared expert computed inside the same launches from its resident bf16
  * tables (gate/up [shared_intermediate, hidden_size], down [hidden_size,

@@ -354,3 +354,25 @@ def test_shared_expert_in_the_launches_refuses_unaligned_operands(operand):
     assert status == _lib.ERR_ARGUMENT
     with pytest.raises(ValueError, match="16-byte aligned"):
         _lib.check(status)
+
+
+@pytest.mark.parametrize("tokens,top_k,local,experts,hidden,inter,rows", [
+    (8, 8, 256, 256, 6144, 2048, 0),         # the decode kernels
+    (9, 8, 256, 256, 6144, 2048, 256),       # fewer than 16 routes an expert
+    (511, 8, 256, 256, 6144, 2048, 256),
+    (512, 8, 256, 256, 6144, 2048, 512),
+    (2048, 8, 32, 256, 6144, 2048, 256),     # a share's one round of items
+    (2730, 8, 64, 256, 6144, 2048, 256),     # exactly two
+    (2800, 8, 64, 256, 6144, 2048, 512),     # more than two
+    (3000, 8, 64, 256, 6144, 2048, 512),
+    (3600, 8, 32, 128, 4096, 1536, 256),
+    (4000, 8, 32, 128, 4096, 1536, 512),
+    (8192, 8, 256, 256, 6144, 1920, 256),    # I not a multiple of 256
+    (8192, 8, 256, 256, 5888, 2048, 256),    # H not a multiple of 512
+    (100, 8, 256, 256, 384, 256, 0),         # H not a multiple of 256: no prefill kernel
+])
+def test_bf16_prefill_stripes(tokens, top_k, local, experts, hidden, inter, rows):
+    # on 256 compute units (this GPU's, and the count without one)
+    from glm_moe import _lib
+
+    assert _lib.lib().glm_moe_prefill_stripe_rows(tokens, top_k, local, experts, hidden, inter) == rows
