@@ -295,8 +295,8 @@ def test_panel_matmul_closed_form_and_invalid_plan(device):
 # Panels as tiles of up to 256 rows: an expert's run of panels ends in every
 # way (one row, one panel, a tile and a row, exact tiles), with unowned experts
 # before and after; 20 experts x 16384 outputs fill 2.5 rounds of 512-row
-# stripes (wide tiles listed twice, FP32 tiles staged in passes); K = 8320 is
-# past the prefill kernel (panel by panel).
+# stripes on 256 CUs (wide tiles listed twice, FP32 tiles staged in passes); K =
+# 8320 is past the prefill kernel (panel by panel).
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("counts,offset,local,n,k", [
     ([5, 300, 33, 1, 513, 64, 31, 0, 256, 40], 1, 8, 768, 640),
@@ -329,6 +329,59 @@ def test_panel_matmul_tiles_match_oracle(device, dtype, counts, offset, local, n
     rows = np.arange(m)
     owned = (rows >= c[:offset].sum()) & (rows < c[:offset + local].sum())
     np.testing.assert_array_equal(got[~owned], 0)
+    if n == 16384:  # the tall stripes' rule, at its line
+        cus = torch.cuda.get_device_properties(device).multi_processor_count
+        assert m >= 16 * local and 2 * max(local, m * 3 // 256) * (n // 512) >= 5 * cus
+
+
+# The same rows through both entry points: tiles (256-row and tall stripes) and,
+# without a workspace, panel by panel.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("counts,offset,local,n,k", [
+    ([5, 300, 33, 1, 513, 64, 31, 0, 256, 40], 1, 8, 768, 640),
+    ([600, 130, 256, 1, 17, 90] + [40] * 14, 0, 20, 16384, 128),
+])
+def test_panel_matmul_tiles_equal_panel_by_panel(device, dtype, counts, offset, local, n, k):
+    from glm_moe import _lib
+    from glm_moe.kernels.fp8_grouped_matmul.panel_kernel import prefill_panel_fp8_matmul
+    from glm_moe.kernels.fp8_grouped_matmul.panels import build_expert_panels
+
+    g = torch.Generator(device=device).manual_seed(n + k)
+    m = sum(counts)
+    x = torch.randn((m, k), generator=g, device=device).to(torch.bfloat16)
+    w = torch.randint(0, 120, (local, n, k), generator=g, device=device, dtype=torch.int32)
+    w = (w + 128 * torch.randint(0, 2, w.shape, generator=g, device=device, dtype=torch.int32)).to(torch.uint8)
+    s = torch.rand((local, n // 128, k // 128), generator=g, device=device)
+    plan = build_expert_panels(torch.tensor(counts, dtype=torch.int32, device=device),
+                               torch.tensor(offset, dtype=torch.int32, device=device), rows=m, local_groups=local)
+    assert _lib.lib().glm_moe_panel_fp8_matmul_workspace_bytes(m, k, local, n) > 0  # on tiles
+    got, _ = prefill_panel_fp8_matmul(x, w, s, plan, result_dtype=dtype)
+    want = torch.full_like(got, float("nan"))
+    _lib.call("glm_moe_panel_fp8_matmul", _lib.ptr(x), m, k, _lib.ptr(w), _lib.ptr(s), local, n,
+              _lib.ptr(plan.expert_ids), _lib.ptr(plan.row_starts), _lib.ptr(plan.live_counts),
+              _lib.ptr(plan.active_panels), plan.expert_ids.numel(), _lib.ptr(plan.owned_rows), _lib.ptr(plan.valid),
+              _lib.F32 if dtype == torch.float32 else _lib.BF16, _lib.ptr(want), _lib.stream_of(x))
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_panel_matmul_tiles_of_an_invalid_plan_are_zero(device, dtype):
+    from glm_moe import _lib
+    from glm_moe.kernels.fp8_grouped_matmul.panel_kernel import prefill_panel_fp8_matmul
+    from glm_moe.kernels.fp8_grouped_matmul.panels import build_expert_panels
+
+    # as test_panel_matmul_closed_form_and_invalid_plan, on a call that runs on tiles
+    m, n, k, local = 1300, 768, 640, 2
+    assert _lib.lib().glm_moe_panel_fp8_matmul_workspace_bytes(m, k, local, n) > 0
+    x = torch.full((m, k), float("nan"), dtype=torch.bfloat16, device=device)
+    w = torch.full((local, n, k), 127, dtype=torch.uint8, device=device)
+    s = torch.full((local, n // 128, k // 128), float("nan"), dtype=torch.float32, device=device)
+    for counts, offset in (([m, 0, 0, 0], 2), ([m, 0, 0, 0], -1), ([m - 1, 0, 0, 0], 0)):
+        p = build_expert_panels(torch.tensor(counts, dtype=torch.int32, device=device),
+                                torch.tensor(offset, dtype=torch.int32, device=device), rows=m, local_groups=local)
+        value, ok = prefill_panel_fp8_matmul(x, w, s, p, result_dtype=dtype)
+        np.testing.assert_array_equal(host_f32(value), 0)
+        assert bool(ok) == (offset == 2)
 
 
 @pytest.mark.parametrize("panels", [20, 1100])  # broken runs: listed by run; more runs than one pass lists: by panel
@@ -716,8 +769,8 @@ def test_decode_step_counts_match_oracle(device, tokens, hidden, inter):
 # Stripe runs: an FP8 prefill work item of the down projection on 256-row
 # stripes runs up to 4 weight stripes of one tile in one continuous ring when K
 # has at least 4 blocks.  H = 1280 gives 5 such stripes (a run of 4, then a
-# run of 1); H = 1536 runs tall stripes (512 rows, one a work item) in both
-# modes.  I = 512 gives K = 4 blocks, where the rings' 3-block look-ahead
+# run of 1); H = 1536 runs tall stripes (512 rows, one a work item) in the
+# FP8 mode and 256-row ones in bf16.  I = 512 gives K = 4 blocks, where the rings' 3-block look-ahead
 # reaches into the next stripe's first blocks; the skewed routing of these
 # seeds gives tiles of every column-group count 1 .. 8 (the 1-2 group bf16
 # tiles run 4-deep rings) and multi-tile experts.
@@ -772,12 +825,13 @@ def test_prefill_work_list_lengths_compute_every_item(device, experts):
     assert ((out.double() - want).abs() <= 2**-6 * scale).all()
 
 
-# Stripe geometries at their edges, both modes: tall down stripes with K = 1
+# Stripe geometries at their edges.  FP8 mode: tall down stripes with K = 1
 # block (I = 128, the two-slot ring's look-ahead past the end from the first
 # block on) beside 256-row gate/up stripes; tall gate/up with K = 2 blocks
 # (H = 256) beside 256-row down stripes; tiles of 5..8 column groups on tall
-# stripes in both projections (~75-120 routes an expert: the half-stage
-# variants of the bf16 kernel, scales of two registers a lane in the FP8 one).
+# stripes in both projections (~75-120 routes an expert, scales of two registers
+# a lane).  The bf16 layers here run 256-row stripes of the same few K blocks and
+# tiles; test_bf16_tall_stripes_* have the tall ones.
 @pytest.mark.parametrize("activations", ["bfloat16", "float8_e4m3fn"])
 @pytest.mark.parametrize("tokens,experts,hidden,inter,top_k,zipf", [
     (200, 16, 512, 128, 4, 0.5),
@@ -900,7 +954,7 @@ def test_prefill_wide_tiles_match_oracle(device, activations, hidden, inter, see
     print(cfg, activations, close(host_f32(out), ref))
 
 
-# Tall stripes of the bf16 kernel: from 16 routes per expert and 2.5 rounds of
+# Tall stripes of the bf16 kernel: from 16 routes per expert and two rounds of
 # gate/up items on 256 CUs, listings (1.5 per 128 routes, at least one per
 # expert) x I / 256.  32 experts with WIDE_COUNTS, I = 2304: 75 x 9 = 675 items,
 # wide tiles of every column-group count as two listings (gate/up K = 4 blocks,
@@ -912,8 +966,11 @@ def test_prefill_wide_tiles_match_oracle(device, activations, hidden, inter, see
     (255, 128, 512, 1280, False),
 ])
 def test_bf16_tall_stripes_match_oracle(device, tokens, experts, hidden, inter, counts):
+    from glm_moe import _lib
     from glm_moe.layers.moe.routed_experts import routed_experts
 
+    assert _lib.lib().glm_moe_prefill_stripe_rows(tokens, 8, experts, experts, hidden, inter) == (
+        256 if tokens == 255 else 512)
     cfg, x, ids, w, tables = _small_case(tokens, experts, hidden, inter, 8, 0.0, seed=tokens + 3)
     if counts:
         rest = tokens * 8 - sum(WIDE_COUNTS)
@@ -925,6 +982,44 @@ def test_bf16_tall_stripes_match_oracle(device, tokens, experts, hidden, inter, 
     ref, ref_ok = O.routed_experts(x, ids, w, **tables)
     assert bool(ok) and ref_ok
     print(cfg, assert_moe_close(host_f32(out), ref))
+
+
+# The least K that tall bf16 stripes meet: down projections of two blocks (I = 256,
+# the whole loop is the two-slot ring's first blocks), 520 experts for two rounds
+# of gate/up items; tiles of 1 .. 8 column groups and wide tiles of each count.
+def test_bf16_tall_stripes_of_two_k_blocks(device):
+    from glm_moe import _lib
+    from glm_moe.layers.moe.routed_experts import routed_experts
+
+    tokens, experts, hidden, inter = 8400, 520, 512, 256
+    assert _lib.lib().glm_moe_prefill_stripe_rows(tokens, 1, experts, experts, hidden, inter) == 512
+    counts = WIDE_COUNTS + [60, 75, 85, 95, 105, 115, 120, 127]
+    rest, more = tokens - sum(counts), experts - len(counts)
+    counts += [rest // more + (i < rest % more) for i in range(more)]
+    g = torch.Generator(device=device).manual_seed(31)
+    ids = torch.repeat_interleave(torch.arange(experts, device=device), torch.tensor(counts, device=device))
+    ids = ids[torch.randperm(tokens, generator=g, device=device)].to(torch.int32)
+    x = torch.randn((tokens, hidden), generator=g, device=device).to(torch.bfloat16)
+
+    def table(n, k):
+        bits = torch.randint(0, 120, (experts, n, k), generator=g, device=device, dtype=torch.int32)
+        bits += 128 * torch.randint(0, 2, bits.shape, generator=g, device=device, dtype=torch.int32)
+        return bits.to(torch.uint8), torch.rand((experts, n // 128, k // 128), generator=g, device=device) * 1e-3 + 1e-3
+
+    tabs = [*table(inter, hidden), *table(inter, hidden), *table(hidden, inter)]
+    out, ok = routed_experts(x, ids[:, None].contiguous(), torch.ones((tokens, 1), device=device), *tabs)
+    assert bool(ok)
+    for e in range(experts):
+        rows = (ids == e).nonzero().squeeze(1)
+        gate_w, up_w, down_w = ((b[e].view(torch.float8_e4m3fn).float()
+                                 * s[e].repeat_interleave(128, 0).repeat_interleave(128, 1)).to(torch.bfloat16).double()
+                                for b, s in zip(tabs[::2], tabs[1::2]))
+        gate, up = ((x[rows].double() @ w.t()).to(torch.bfloat16).double() for w in (gate_w, up_w))
+        act = ((gate * torch.sigmoid(gate).to(torch.bfloat16).double()).to(torch.bfloat16).double() * up).to(
+            torch.bfloat16).double()
+        # bf16 rounding of gate, up, the SwiGLU and the row, each 2**-9 of its value
+        bound = 2**-6 * (act.abs() @ down_w.abs().t())
+        assert ((out[rows].double() - act @ down_w.t()).abs() <= bound).all(), e
 
 
 def test_routed_experts_invalid_routes_follow_reference(device):
