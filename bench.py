@@ -255,15 +255,16 @@ def full_layer(work, steps, warmup):
     """The whole MoE layer (K calls replayed from one HIP graph), as the reference's layer bodies compute it: the bf16
     shared expert (random-init N(0, 0.02) weights of the contract's shape,
     I_shared = I) and the routed experts with the epilogue
-    bf16(bf16(routed * 2.5) + shared) fused into their route-sum kernel.  On
-    decode shapes the shared expert runs inside the two decode kernels
-    (glm_moe_moe_layer_resident); for 2-8 rows in the few-row shared-expert
-    kernels (glm_moe_shared_expert_rows); else as torch GEMMs on hipBLASLt.
+    bf16(bf16(routed * 2.5) + shared) fused into their route-sum kernel.  bf16
+    layers run prefill_moe_from_routes, which puts the shared expert inside the
+    two decode kernels for up to 8 rows, inside the two prefill launches for up
+    to 6144, and on hipBLASLt above; in the FP8 mode it runs on hipBLASLt.
     Returns (us per layer, algorithmic bytes of the shared expert, how)."""
     import torch
 
-    from glm_moe.layers.moe.routed_experts import (_shared_expert, routed_experts, shared_expert_rows_fit,
-                                                   uses_decode_kernels)
+    from glm_moe.contracts import single_gpu_contract
+    from glm_moe.layers.moe.routed_experts import (_shared_expert, _shared_in_prefill, prefill_moe_from_routes,
+                                                   routed_experts, uses_decode_kernels)
 
     cfg = work.cfg
     device = work.inputs[0][0].device
@@ -277,15 +278,14 @@ def full_layer(work, steps, warmup):
     out = torch.empty((cfg.tokens, cfg.hidden), dtype=torch.bfloat16, device=device)
     n_rot = len(work.inputs)
 
-    # up to 8 rows on the decode kernels: the shared expert inside them (one row: the
-    # decode body); more: hipBLASLt (each reads the shared weights once)
-    resident = work.activations == "bfloat16" and cfg.tokens <= 8 and uses_decode_kernels(
-        cfg.tokens, cfg.top_k, cfg.hidden, cfg.intermediate)
+    bf16 = work.activations == "bfloat16"
+    contract = single_gpu_contract(hidden_size=cfg.hidden, intermediate_size=cfg.intermediate,
+                                   num_experts=cfg.experts, top_k=cfg.top_k)
 
     def layer(i):
         x, ids, w = work.inputs[i % n_rot]
-        if resident:
-            routed_experts(x, ids, w, *tables, out=out, shared_tables=(sg, su, sd), routed_scale=2.5)
+        if bf16:
+            prefill_moe_from_routes(x, ids, w, *tables, sg, su, sd, contract=contract)
         else:
             shared = _shared_expert(x, sg, su, sd)
             routed_experts(x, ids, w, *tables, out=out, shared=shared, routed_scale=2.5,
@@ -293,11 +293,11 @@ def full_layer(work, steps, warmup):
 
     ms, _ = graph_time(layer, steps, warmup)
     shared_bytes = 3 * inter_shared * cfg.hidden * 2
-    if resident:
+    if bf16 and cfg.tokens <= 8 and uses_decode_kernels(cfg.tokens, cfg.top_k, cfg.hidden, cfg.intermediate):
         how = ("shared expert inside the two decode kernels (glm_moe_moe_layer_resident"
                + (")" if cfg.tokens == 1 else "; routes grouped by expert, shared rows streamed once per token group)"))
-    elif shared_expert_rows_fit(cfg.tokens, cfg.hidden, inter_shared):
-        how = "shared expert on the few-row kernels (glm_moe_shared_expert_rows), epilogue fused (glm_moe_moe_layer)"
+    elif bf16 and _shared_in_prefill(work.inputs[0][0], (sg, su, sd), cfg.top_k, cfg.experts):
+        how = "shared expert inside the two prefill launches (glm_moe_moe_layer_shared)"
     else:
         how = "shared expert on torch/hipBLASLt GEMMs and the library SwiGLU kernel, epilogue fused (glm_moe_moe_layer)"
     return ms * 1e3, shared_bytes, how
