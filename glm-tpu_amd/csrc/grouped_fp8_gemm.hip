@@ -1,5 +1,9 @@
-// Route-grouped FP8 expert projection on gfx950 bf16 MFMA: the skinny
-// (decode) kernel, for work tiles of at most 4, 16 or 32 routes.
+// Route-grouped FP8 expert projection on gfx950 bf16 MFMA: the skinny kernel,
+// for work tiles of at most 4, 16 or 32 routes.  It takes what the decode and
+// prefill kernels do not: layers of more than 64 routes whose geometry does not
+// fit the prefill kernel, routed projections with K above 8192 or unaligned
+// tensors, and panel matmuls that are small, unaligned or past the prefill
+// kernel's geometry.
 //
 // Computes, for every work tile (expert e, sorted routes [r0, r0 + live)) and
 // every BN-row stripe of the expert's weight table,

@@ -558,8 +558,9 @@ __device__ __forceinline__ void shared_item_run(const GroupedGemmArgs& a, uint8_
 }
 
 // Rows of the shared expert's tiles: up to 256, and two tiles of up to 128 for
-// fewer rows, so that an XCD's workgroups of a 16-stripe projection are a
-// multiple of its 4 shader engines, which take them in turn.
+// fewer rows, so that an XCD's workgroups of a 16-stripe projection (gate/up of
+// I = 2048) are a multiple of its 4 shader engines, which take them in turn (the
+// 24 down stripes of H = 6144 give an XCD 6 workgroups instead of 3).
 __host__ __device__ __forceinline__ int shared_tile_rows(int rows) {
   return rows > 256 ? 256 : (rows + 31) / 32 * 16;
 }

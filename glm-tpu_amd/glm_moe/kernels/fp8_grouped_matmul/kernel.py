@@ -2,12 +2,13 @@
 
 Mirrors ``glm_tpu/kernels/fp8_grouped_matmul/kernel.py``:
 ``RoutedProjectionConfig`` (``:53-94``) and ``fp8_routed_projection``
-(``:125-299``).  On the GPU the owned slots become one-row work tiles of the
-grouped gfx950 kernel (split-K over four waves); each selected expert's
-weights are streamed once from HBM with 128-bit loads, decoded per 128x128
-block in registers to bf16 and multiplied on MFMA with FP32 accumulation.
-The TPU tile sizes of the config are validated for signature parity; the GPU
-kernel picks its own tiling.
+(``:125-299``).  On the GPU a workgroup computes 16 weight rows of every table
+for one slot, or for two slots of one expert, its four waves splitting K: the
+weights are streamed with 128-bit loads, decoded per 128x128 block in registers
+to bf16 and multiplied with v_dot2 in FP32, all in one launch.  K above 8192 and
+tensors that are not 16-byte aligned run as one-row tiles of the grouped kernel
+(MFMA, split-K over four waves) instead.  The TPU tile sizes of the config are
+validated for signature parity; the GPU kernel picks its own tiling.
 """
 
 from __future__ import annotations

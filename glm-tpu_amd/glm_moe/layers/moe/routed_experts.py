@@ -250,8 +250,9 @@ def routed_experts(
     and ``valid`` also requires a finite output (``:126``).  ``shared_tables``
     (its resident bf16 gate, up, down tables) instead computes the shared
     expert inside the same two decode kernels (decode shapes only:
-    ``uses_decode_kernels``); it streams the shared weights once per row, so
-    the layer bodies use it for a single row.
+    ``uses_decode_kernels``); gate/up streams the shared weights once per group
+    of up to 4 rows, down once, and the layer bodies use it for up to
+    ``RESIDENT_ROWS_MAX`` rows.
     """
     if hidden.ndim != 2 or hidden.dtype != torch.bfloat16:
         raise ValueError("routed experts take bf16 [tokens, hidden] rows")
@@ -592,10 +593,15 @@ def _prefill_shared_bytes(tokens: int, top_k: int, experts: int, hidden: int, in
 def _shared_in_prefill(hidden: torch.Tensor, tables, top_k: int, experts: int) -> bool:
     """Whether the layer's prefill launches compute the shared expert too.
 
-    Up to SHARED_PREFILL_ROWS_MAX rows: GLM-5 shape, T = 9 / 61 / 128 / 777 /
-    2048 / 4000: 417 / 1042 / 1278 / 1760 / 2281 / 3385 us with the shared
-    expert's GEMMs on hipBLASLt, 387 / 1020 / 1243 / 1694 / 2252 / 3362 with its
-    rows inside; at T = 8000 its GEMMs are large enough (5667 against 5689).
+    Up to SHARED_PREFILL_ROWS_MAX rows.  GLM-5 shape, T = 9 / 128 / 600 / 2000 /
+    4000: 385 / 1272 / 1624 / 2207 / 3316 us with the shared expert's GEMMs on
+    hipBLASLt, 358 / 1237 / 1577 / 2188 / 3275 with its rows inside; from 5000
+    rows on the two are within 1 % (6000: 4478, 4468; 8000: 5554, 5589), so the
+    line there is worth nothing either way.  Nine other shapes (8 to 128 experts,
+    H 1024 to 6144, top-2 to 8, even and skewed): 0.38 to 1.19 of the GEMMs' time
+    below 4500 rows, 0.89 in the mean, small layers the most; slower only where
+    the routed items just fill whole rounds of the CUs (16 experts of 6144 x
+    2048, top-2, T = 300: 189, 224); 0.83 to 1.03 from 5000 to 8000 rows.
     """
     rows, h = hidden.shape
     return (rows <= SHARED_PREFILL_ROWS_MAX
